@@ -28,9 +28,11 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdint>
+#include <cstring>
 
 #include "nibble_kv.hpp"
 #include "nibble_page.hpp"
+#include "nibble_work.hpp"
 
 namespace cfnib {
 
@@ -252,18 +254,20 @@ __device__ inline Visible visible_range(uint32_t qpos, uint32_t window, uint32_t
 }
 
 template <int LG, int G>
-__global__ __launch_bounds__(256) void nib_attn_kernel(const AttnItem *__restrict__ items, AttnShape sh, uint32_t hw,
-                                                       uint32_t hgroups, uint32_t qchunks, float *__restrict__ ws) {
-  const AttnItem &it = items[blockIdx.z];
-  const uint32_t split = blockIdx.x;
-  if (split >= it.nsplit) return;
-  // splits [0, vbase) are the MFMA kernel's, then vsplits page splits of this kernel, then the active page
+__global__ __launch_bounds__(256) void nib_attn_kernel(const AttnItem *__restrict__ items, WorkList work, AttnShape sh,
+                                                       uint32_t hw, uint32_t hgroups, uint32_t qchunks,
+                                                       float *__restrict__ ws) {
+  const uint32_t ii = work_item(work.first, work.items, blockIdx.x);
+  const AttnItem &it = items[ii];
+  // splits [0, vbase) are the MFMA kernel's, then vsplits page splits of this kernel, then asplits over the active
+  // page; an item with nothing visible has one (empty) split
   const uint32_t vbase = it.mfma_nb ? it.page_splits : 0u;
-  if (split < vbase) return;  // the MFMA kernel reads these pages
+  const uint32_t mine_n = it.nsplit - vbase;  // this kernel's splits of the item (at least 1 where it owns units)
+  const uint32_t local = blockIdx.x - work.first[ii];
+  const uint32_t y = local / mine_n, split = vbase + (local - y * mine_n);
   const uint32_t per_tok = hgroups * qchunks;
-  const uint32_t qt = blockIdx.y / per_tok;
-  if (qt >= it.q_tokens) return;
-  const uint32_t rest = blockIdx.y - qt * per_tok;
+  const uint32_t qt = y / per_tok;
+  const uint32_t rest = y - qt * per_tok;
   const uint32_t hg = rest / qchunks;
   const uint32_t qc = rest - hg * qchunks;
   const uint32_t unit = threadIdx.x / LG;
@@ -380,23 +384,30 @@ __global__ __launch_bounds__(256) void nib_attn_kernel(const AttnItem *__restric
         }
       }
     }
-  } else {  // the active fp32 page
-    const uint32_t n = it.active_count;
-    for (uint32_t tok = 0; tok < n; ++tok) {
-      float kf[8], vf[8];
-      if (lane_ok) {
-        const uint64_t base = (uint64_t(tok) * kvh + h) * D + 8u * c;
-        const float4 a = *reinterpret_cast<const float4 *>(it.active_k + base);
-        const float4 b = *reinterpret_cast<const float4 *>(it.active_k + base + 4);
-        const float4 x = *reinterpret_cast<const float4 *>(it.active_v + base);
-        const float4 y = *reinterpret_cast<const float4 *>(it.active_v + base + 4);
-        kf[0] = a.x; kf[1] = a.z; kf[2] = b.x; kf[3] = b.z; kf[4] = a.y; kf[5] = a.w; kf[6] = b.y; kf[7] = b.w;
-        vf[0] = x.x; vf[1] = x.z; vf[2] = y.x; vf[3] = y.z; vf[4] = x.y; vf[5] = x.w; vf[6] = y.y; vf[7] = y.w;
-      } else {
+  } else {  // kActiveTokens tokens of the active fp32 page, four tokens' loads in flight together
+    const uint32_t a0 = (split - vbase - it.vsplits) * kActiveTokens;
+    const uint32_t n = min(it.active_count, a0 + kActiveTokens);
+    for (uint32_t t0 = a0; t0 < n; t0 += 4u) {
+      float4 ka[4], kb[4], va[4], vb[4];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) kf[e] = vf[e] = 0.0f;
+      for (int u = 0; u < 4; ++u) {
+        const float4 z = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        ka[u] = kb[u] = va[u] = vb[u] = z;
+        if (lane_ok) {  // past the end: the last token again (not consumed)
+          const uint64_t base = (uint64_t(min(t0 + u, n - 1u)) * kvh + h) * D + 8u * c;
+          ka[u] = *reinterpret_cast<const float4 *>(it.active_k + base);
+          kb[u] = *reinterpret_cast<const float4 *>(it.active_k + base + 4);
+          va[u] = *reinterpret_cast<const float4 *>(it.active_v + base);
+          vb[u] = *reinterpret_cast<const float4 *>(it.active_v + base + 4);
+        }
       }
-      consume<LG, G>(st, qv, qsum, kf, 1.0f, 0.0f, vf, 1.0f, 0.0f, key_visible(it.active_begin + tok), scale_log2);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        if (t0 + u >= n) break;  // uniform across the workgroup
+        const float kf[8] = {ka[u].x, ka[u].z, kb[u].x, kb[u].z, ka[u].y, ka[u].w, kb[u].y, kb[u].w};
+        const float vf[8] = {va[u].x, va[u].z, vb[u].x, vb[u].z, va[u].y, va[u].w, vb[u].y, vb[u].w};
+        consume<LG, G>(st, qv, qsum, kf, 1.0f, 0.0f, vf, 1.0f, 0.0f, key_visible(it.active_begin + t0 + u), scale_log2);
+      }
     }
   }
 
@@ -421,12 +432,17 @@ __global__ __launch_bounds__(256) void nib_attn_kernel(const AttnItem *__restric
   }
 }
 
-// One wave per (query head, query token, item): combine the splits and store the normalised row.
-__global__ __launch_bounds__(64) void nib_merge_kernel(const AttnItem *__restrict__ items, AttnShape sh,
-                                                       const float *__restrict__ ws) {
-  const AttnItem &it = items[blockIdx.z];
-  const uint32_t qt = blockIdx.y, qh = blockIdx.x, lane = threadIdx.x;
-  if (qt >= it.q_tokens) return;
+// One wave per (query head, query token) row of an item (the units of `work`): combine the splits and store the
+// normalised row.
+constexpr uint32_t kMergeRows = 4;  // rows (waves) per workgroup
+__global__ __launch_bounds__(64 * kMergeRows) void nib_merge_kernel(const AttnItem *__restrict__ items, WorkList work,
+                                                                    AttnShape sh, const float *__restrict__ ws) {
+  const uint32_t unit = __builtin_amdgcn_readfirstlane(blockIdx.x * kMergeRows + (threadIdx.x >> 6));
+  if (unit >= work.total) return;
+  const uint32_t ii = work_item(work.first, work.items, unit);
+  const AttnItem &it = items[ii];
+  const uint32_t local = unit - work.first[ii], lane = threadIdx.x & 63u;
+  const uint32_t qt = local / sh.q_heads, qh = local - qt * sh.q_heads;
   const uint32_t D = sh.head_dim, stride = D + 4u;
   const float *row0 = ws + it.ws_offset + (uint64_t(qt) * sh.q_heads + qh) * stride;
   const uint64_t split_stride = uint64_t(it.q_tokens) * sh.q_heads * stride;
@@ -480,19 +496,19 @@ __global__ __launch_bounds__(64) void nib_merge_kernel(const AttnItem *__restric
 }
 
 template <int LG, int G>
-hipError_t launch_attn_lg_g(dim3 grid, dim3 block, hipStream_t s, const AttnItem *items, const AttnShape &sh,
-                            uint32_t hw, uint32_t hgroups, uint32_t qchunks, float *ws) {
-  nib_attn_kernel<LG, G><<<grid, block, 0, s>>>(items, sh, hw, hgroups, qchunks, ws);
+hipError_t launch_attn_lg_g(const WorkList &work, dim3 block, hipStream_t s, const AttnItem *items,
+                            const AttnShape &sh, uint32_t hw, uint32_t hgroups, uint32_t qchunks, float *ws) {
+  nib_attn_kernel<LG, G><<<work.total, block, 0, s>>>(items, work, sh, hw, hgroups, qchunks, ws);
   return hipPeekAtLastError();
 }
 
 template <int LG>
-hipError_t launch_attn_lg(uint32_t G, dim3 grid, dim3 block, hipStream_t s, const AttnItem *items,
+hipError_t launch_attn_lg(uint32_t G, const WorkList &work, dim3 block, hipStream_t s, const AttnItem *items,
                           const AttnShape &sh, uint32_t hw, uint32_t hgroups, uint32_t qchunks, float *ws) {
   switch (G) {
-    case 1: return launch_attn_lg_g<LG, 1>(grid, block, s, items, sh, hw, hgroups, qchunks, ws);
-    case 2: return launch_attn_lg_g<LG, 2>(grid, block, s, items, sh, hw, hgroups, qchunks, ws);
-    default: return launch_attn_lg_g<LG, 4>(grid, block, s, items, sh, hw, hgroups, qchunks, ws);
+    case 1: return launch_attn_lg_g<LG, 1>(work, block, s, items, sh, hw, hgroups, qchunks, ws);
+    case 2: return launch_attn_lg_g<LG, 2>(work, block, s, items, sh, hw, hgroups, qchunks, ws);
+    default: return launch_attn_lg_g<LG, 4>(work, block, s, items, sh, hw, hgroups, qchunks, ws);
   }
 }
 
@@ -566,7 +582,7 @@ hipError_t AttnRunner::run(const std::vector<AttnRequest> &reqs, const AttnShape
 
   std::vector<AttnItem> items(reqs.size());
   uint64_t floats = 0;
-  uint32_t max_split = 1, max_qtok = 1, max_mfma_split = 0;
+  uint32_t max_split = 1, max_qtok = 1;
   bool any_nb[5] = {false, false, false, false, false};
   const uint32_t wave_lanes = std::min(64u, hw * lg);  // lanes of the VALU kernel's first wave
   for (size_t i = 0; i < reqs.size(); ++i) {
@@ -590,7 +606,6 @@ hipError_t AttnRunner::run(const std::vector<AttnRequest> &reqs, const AttnShape
       const uint32_t tiles = (r.page_count * cpp + 3u) / 4u;
       it.units_per_split = tps;
       it.page_splits = (tiles + tps - 1u) / tps;
-      max_mfma_split = std::max(max_mfma_split, it.page_splits);
       any_nb[nb[i]] = true;
       it.vunits = nb[i] == kMfmaContract ? wave_lanes : 0u;  // one lane per page tests it
       it.vsplits = it.vunits ? (r.page_count + it.vunits - 1u) / it.vunits : 0u;
@@ -610,7 +625,8 @@ hipError_t AttnRunner::run(const std::vector<AttnRequest> &reqs, const AttnShape
     it.window = r.window;
     it.scale_log2 = r.softmax_scale * 1.4426950408889634f;
     it.flags = r.flags;
-    it.nsplit = (it.mfma_nb ? it.page_splits : 0u) + it.vsplits + (it.active_count > 0u ? 1u : 0u);
+    it.asplits = (it.active_count + kActiveTokens - 1u) / kActiveTokens;
+    it.nsplit = (it.mfma_nb ? it.page_splits : 0u) + it.vsplits + it.asplits;
     if (it.nsplit == 0u) it.nsplit = 1u;  // nothing visible: one empty split, the row comes out 0
     it.ws_offset = floats;
     floats += uint64_t(it.nsplit) * it.q_tokens * sh.q_heads * (D + 4u);
@@ -622,7 +638,38 @@ hipError_t AttnRunner::run(const std::vector<AttnRequest> &reqs, const AttnShape
     error = "attention batch exceeds the launch grid (too many query tokens or items in one call)";
     return hipErrorInvalidValue;
   }
-  const uint64_t table_bytes = (items.size() * sizeof(AttnItem) + 255u) & ~uint64_t(255);
+  // the launches' work lists (prefix sums of their items' workgroups), uploaded behind the items: the VALU kernel's,
+  // the merge's, then one per MFMA mode in use
+  const size_t n = items.size();
+  std::vector<uint32_t> modes;
+  for (uint32_t m : {1u, 2u, kMfmaContract, 4u})
+    if (any_nb[m]) modes.push_back(m);
+  const size_t lists = 2 + modes.size();
+  const uint64_t list_at = (n * sizeof(AttnItem) + 255u) & ~uint64_t(255);
+  std::vector<char> table(list_at + lists * (n + 1) * sizeof(uint32_t));
+  std::memcpy(table.data(), items.data(), n * sizeof(AttnItem));
+  std::vector<uint32_t> totals(lists);
+  for (size_t l = 0; l < lists; ++l) {
+    uint32_t *first = reinterpret_cast<uint32_t *>(table.data() + list_at) + l * (n + 1);
+    uint64_t at = 0;
+    for (size_t i = 0; i <= n; ++i) {
+      if (at > 0x7fffffffu) {
+        error = "attention batch exceeds the launch grid (too many query tokens or items in one call)";
+        return hipErrorInvalidValue;
+      }
+      first[i] = static_cast<uint32_t>(at);
+      if (i == n) break;
+      const AttnItem &it = items[i];
+      if (l == 0)
+        at += uint64_t(it.nsplit - (it.mfma_nb ? it.page_splits : 0u)) * it.q_tokens * hgroups * qchunks;
+      else if (l == 1)
+        at += uint64_t(it.q_tokens) * sh.q_heads;
+      else if (it.mfma_nb == modes[l - 2])
+        at += nib_mfma_workgroups(it, sh);
+    }
+    totals[l] = static_cast<uint32_t>(at);
+  }
+  const uint64_t table_bytes = (table.size() + 255u) & ~uint64_t(255);
   const uint64_t need = table_bytes + floats * sizeof(float);
   if (need > bytes_) {
     if (ws_) {
@@ -641,30 +688,28 @@ hipError_t AttnRunner::run(const std::vector<AttnRequest> &reqs, const AttnShape
     }
     bytes_ = grow;
   }
-  hipError_t e = hipMemcpyAsync(ws_, items.data(), items.size() * sizeof(AttnItem), hipMemcpyHostToDevice, stream);
+  hipError_t e = hipMemcpyAsync(ws_, table.data(), table.size(), hipMemcpyHostToDevice, stream);
   if (e != hipSuccess) return e;
   const AttnItem *d_items = static_cast<const AttnItem *>(ws_);
   float *partials = reinterpret_cast<float *>(static_cast<char *>(ws_) + table_bytes);
-  const dim3 grid(max_split, static_cast<uint32_t>(ydim), static_cast<uint32_t>(items.size()));
+  const uint32_t *d_lists = reinterpret_cast<const uint32_t *>(static_cast<const char *>(ws_) + list_at);
+  auto work = [&](size_t l) { return WorkList{d_lists + l * (n + 1), static_cast<uint32_t>(n), totals[l]}; };
   const dim3 block(hw * lg);
   // the VALU kernel serves items without the MFMA path, every active page and every item with nothing visible
-  bool valu_work = false;
-  for (const AttnItem &it : items) valu_work = valu_work || !it.mfma_nb || it.nsplit > it.page_splits;
-  if (valu_work) switch (lg) {
-    case 4: e = launch_attn_lg<4>(G, grid, block, stream, d_items, sh, hw, hgroups, qchunks, partials); break;
-    case 8: e = launch_attn_lg<8>(G, grid, block, stream, d_items, sh, hw, hgroups, qchunks, partials); break;
-    case 16: e = launch_attn_lg<16>(G, grid, block, stream, d_items, sh, hw, hgroups, qchunks, partials); break;
-    default: e = launch_attn_lg<32>(G, grid, block, stream, d_items, sh, hw, hgroups, qchunks, partials); break;
+  if (totals[0]) switch (lg) {
+    case 4: e = launch_attn_lg<4>(G, work(0), block, stream, d_items, sh, hw, hgroups, qchunks, partials); break;
+    case 8: e = launch_attn_lg<8>(G, work(0), block, stream, d_items, sh, hw, hgroups, qchunks, partials); break;
+    case 16: e = launch_attn_lg<16>(G, work(0), block, stream, d_items, sh, hw, hgroups, qchunks, partials); break;
+    default: e = launch_attn_lg<32>(G, work(0), block, stream, d_items, sh, hw, hgroups, qchunks, partials); break;
   }
   if (e != hipSuccess) return e;
-  for (uint32_t n : {1u, 2u, kMfmaContract, 4u}) {
-    if (!any_nb[n]) continue;
-    e = launch_nib_mfma(n, d_items, static_cast<uint32_t>(items.size()), max_mfma_split, max_qtok, sh, partials,
-                        stream);
+  for (size_t m = 0; m < modes.size(); ++m) {
+    e = launch_nib_mfma(modes[m], d_items, work(2 + m), sh, partials, stream);
     if (e != hipSuccess) return e;
   }
-  nib_merge_kernel<<<dim3(sh.q_heads, max_qtok, static_cast<uint32_t>(items.size())), 64, 0, stream>>>(d_items, sh,
-                                                                                                     partials);
+  if (totals[1])
+    nib_merge_kernel<<<(totals[1] + kMergeRows - 1u) / kMergeRows, 64 * kMergeRows, 0, stream>>>(d_items, work(1), sh,
+                                                                                                 partials);
   e = hipPeekAtLastError();
   if (e == hipSuccess) launches_ = 2;
   return e;

@@ -30,6 +30,7 @@
 #include "cf_device.hpp"
 #include "nibble_kv.hpp"
 #include "nibble_page.hpp"
+#include "nibble_work.hpp"
 
 namespace cfnib {
 namespace {
@@ -113,7 +114,7 @@ __device__ inline void wave_sync_lds() {
 // an inclusive window): each page's own block size (a multiple of 32) gives one scale per 32-dim quarter of a row,
 // and pages that mfma_page_ok refuses are left to the VALU kernel.
 template <int MODE>
-__global__ __launch_bounds__(256) void nib_mfma_kernel(const AttnItem *__restrict__ items, AttnShape sh,
+__global__ __launch_bounds__(256) void nib_mfma_kernel(const AttnItem *__restrict__ items, WorkList work, AttnShape sh,
                                                        uint32_t qchunks, float *__restrict__ ws) {
   constexpr bool PG = MODE == static_cast<int>(kMfmaContract);
   constexpr int NB = PG ? 4 : MODE;
@@ -121,15 +122,15 @@ __global__ __launch_bounds__(256) void nib_mfma_kernel(const AttnItem *__restric
   __shared__ __attribute__((aligned(16))) uint8_t s_kv[kWaves][2][2][kTileBytes];  // [wave][buffer][K, V]
   __shared__ __attribute__((aligned(16))) float s_p[kWaves][4][64];                // p per [head][slot]
   __shared__ float s_vs[kWaves][64][NB];                                           // V scales per slot
-  const AttnItem &it = items[blockIdx.z];
-  if (it.mfma_nb != static_cast<uint32_t>(MODE)) return;
-  const uint32_t split = blockIdx.x;
-  if (split >= it.page_splits) return;
+  const uint32_t ii = work_item(work.first, work.items, blockIdx.x);
+  const AttnItem &it = items[ii];
+  // the item's workgroups: split fastest, then the chunk of query heads, the KV head, the query token
+  const uint32_t local = blockIdx.x - work.first[ii];
   const uint32_t kvh = sh.kv_heads, gqa = sh.gqa;
+  const uint32_t y = local / it.page_splits, split = local - y * it.page_splits;
   const uint32_t per_tok = qchunks * kvh;
-  const uint32_t qt = blockIdx.y / per_tok;
-  if (qt >= it.q_tokens) return;
-  const uint32_t rest = blockIdx.y - qt * per_tok;
+  const uint32_t qt = y / per_tok;
+  const uint32_t rest = y - qt * per_tok;
   const uint32_t h = rest / qchunks, qc = rest - h * qchunks;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int G = lane >> 4, t = lane & 15;
@@ -460,18 +461,20 @@ __global__ __launch_bounds__(256) void nib_mfma_kernel(const AttnItem *__restric
 
 }  // namespace
 
-hipError_t launch_nib_mfma(uint32_t nb, const AttnItem *items, uint32_t nitems, uint32_t max_page_splits,
-                           uint32_t max_qtok, const AttnShape &sh, float *ws, hipStream_t stream) {
-  if (sh.head_dim != kD || max_page_splits == 0) return hipSuccess;
+uint64_t nib_mfma_workgroups(const AttnItem &it, const AttnShape &sh) {
+  return uint64_t(it.page_splits) * it.q_tokens * ((sh.gqa + 3u) / 4u) * sh.kv_heads;
+}
+
+hipError_t launch_nib_mfma(uint32_t nb, const AttnItem *items, const WorkList &work, const AttnShape &sh, float *ws,
+                           hipStream_t stream) {
+  if (sh.head_dim != kD || work.total == 0) return hipSuccess;
   const uint32_t qchunks = (sh.gqa + 3u) / 4u;
-  const uint64_t ydim = uint64_t(max_qtok) * qchunks * sh.kv_heads;
-  if (ydim > 65535u) return hipErrorInvalidValue;
-  const dim3 grid(max_page_splits, static_cast<uint32_t>(ydim), nitems);
+  const dim3 grid(work.total);
   switch (nb) {
-    case 1: nib_mfma_kernel<1><<<grid, 256, 0, stream>>>(items, sh, qchunks, ws); break;
-    case 2: nib_mfma_kernel<2><<<grid, 256, 0, stream>>>(items, sh, qchunks, ws); break;
-    case kMfmaContract: nib_mfma_kernel<kMfmaContract><<<grid, 256, 0, stream>>>(items, sh, qchunks, ws); break;
-    default: nib_mfma_kernel<4><<<grid, 256, 0, stream>>>(items, sh, qchunks, ws); break;
+    case 1: nib_mfma_kernel<1><<<grid, 256, 0, stream>>>(items, work, sh, qchunks, ws); break;
+    case 2: nib_mfma_kernel<2><<<grid, 256, 0, stream>>>(items, work, sh, qchunks, ws); break;
+    case kMfmaContract: nib_mfma_kernel<kMfmaContract><<<grid, 256, 0, stream>>>(items, work, sh, qchunks, ws); break;
+    default: nib_mfma_kernel<4><<<grid, 256, 0, stream>>>(items, work, sh, qchunks, ws); break;
   }
   return hipPeekAtLastError();
 }
