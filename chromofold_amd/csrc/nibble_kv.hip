@@ -32,6 +32,7 @@
 
 #include "nibble_kv.hpp"
 #include "nibble_page.hpp"
+#include "nibble_query.hpp"
 #include "nibble_work.hpp"
 
 namespace cfnib {
@@ -242,25 +243,14 @@ __device__ inline void consume(RowState<G> &st, const float (&qv)[G][8], const f
   }
 }
 
-// Visible positions [lo, hi] of query position qpos: p <= q and, with a window, p + window > q; with kOpenWindow
-// every p except those with window > 0 and p + window < q.
-struct Visible {
-  uint32_t lo, hi;
-  __device__ bool operator()(uint32_t pos) const { return pos >= lo && pos <= hi; }
-};
-__device__ inline Visible visible_range(uint32_t qpos, uint32_t window, uint32_t flags) {
-  if (flags & kOpenWindow) return {window != 0u && qpos >= window ? qpos - window : 0u, 0xFFFFFFFFu};
-  return {window != 0u && qpos >= window ? qpos - window + 1u : 0u, qpos};
-}
-
 template <int LG, int G>
 __global__ __launch_bounds__(256) void nib_attn_kernel(const AttnItem *__restrict__ items, WorkList work, AttnShape sh,
                                                        uint32_t hw, uint32_t hgroups, uint32_t qchunks,
                                                        float *__restrict__ ws) {
   const uint32_t ii = work_item(work.first, work.items, blockIdx.x);
   const AttnItem &it = items[ii];
-  // splits [0, vbase) are the MFMA kernel's, then vsplits page splits of this kernel, then asplits over the active
-  // page; an item with nothing visible has one (empty) split
+  // splits [0, vbase) are the MFMA kernel's (which takes its items' active pages along), then vsplits page splits of
+  // this kernel, then asplits over the active page; an item with nothing visible has one (empty) split
   const uint32_t vbase = it.mfma_nb ? it.page_splits : 0u;
   const uint32_t mine_n = it.nsplit - vbase;  // this kernel's splits of the item (at least 1 where it owns units)
   const uint32_t local = blockIdx.x - work.first[ii];
@@ -283,16 +273,27 @@ __global__ __launch_bounds__(256) void nib_attn_kernel(const AttnItem *__restric
   const uint32_t sx = (flags & kSignedNibbles) ? 0x88888888u : 0u;  // n ^ 8 - 8 is the two's-complement value
 
   float qv[G][8], qsum[G];
+  {
+    uint64_t off[G];
+    bool ok[G];  // (the other lanes read the item's first query row and drop it)
 #pragma unroll
-  for (int j = 0; j < G; ++j) {
-    const bool ok = lane_ok && j0 + j < gqa;
-    const uint64_t qoff = uint64_t(qt) * it.q_token_stride + uint64_t(h * gqa + j0 + j) * it.q_head_stride;
-    qsum[j] = 0.0f;
+    for (int j = 0; j < G; ++j) {
+      ok[j] = lane_ok && j0 + j < gqa;
+      off[j] = ok[j] ? uint64_t(qt) * it.q_token_stride + uint64_t(h * gqa + j0 + j) * it.q_head_stride +
+                           uint64_t(8u * c) * it.q_elem_stride
+                     : 0u;
+    }
+    float x[G][8];
+    const bool packed = ((reinterpret_cast<uintptr_t>(it.q) | it.q_token_stride | it.q_head_stride) & 15u) == 0u;
+    load_rows8<G>(x, it.q, it.q_type, off, it.q_elem_stride, packed);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float x = ok ? load_scalar(it.q, it.q_type, qoff + uint64_t(8u * c + e) * it.q_elem_stride) : 0.0f;
-      qv[j][nib_pos(e)] = x;
-      qsum[j] += x;
+    for (int j = 0; j < G; ++j) {
+      qsum[j] = 0.0f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        qv[j][nib_pos(e)] = ok[j] ? x[j][e] : 0.0f;
+        qsum[j] += qv[j][nib_pos(e)];
+      }
     }
   }
   RowState<G> st;
@@ -572,13 +573,21 @@ hipError_t AttnRunner::run(const std::vector<AttnRequest> &reqs, const AttnShape
     // head_dim is 128 and pages have a planned size; other flagged requests stay on the VALU kernel
     nb[i] = r.flags == kContractFlags ? (D == 128u && cpp > 0u ? kMfmaContract : 0u)
                                       : r.flags ? 0u : mfma_sets(D, r.block_size);
+    // the MFMA kernel's offsets inside a page's payload (64 bytes per token and KV head) are 32-bit
+    if (uint64_t(16u) * cpp * sh.kv_heads * 64u > 0xFFFFFFFFull) nb[i] = 0u;
     if (nb[i]) tile_work += uint64_t((r.page_count * cpp + 3u) / 4u) * r.query.token_count * ((sh.gqa + 3u) / 4u);
     else page_work += uint64_t(r.page_count) * r.query.token_count * hgroups * qchunks;
   }
   const uint32_t pps = static_cast<uint32_t>(std::clamp<uint64_t>((page_work + 2047u) / 2048u, 1u, 64u));
-  // the MFMA kernel's workgroups take four 64-slot tiles per round (one per wave), KV head by KV head
+  // The MFMA kernel's workgroups take four 64-slot tiles per round (one per wave), KV head by KV head. A batch of up to
+  // about 8 tiles a wave gets one round of workgroups (three fit a CU; 512 leaves room for the last splits of the
+  // items): a workgroup's prologue and merge cost as much as two or three tiles (26 items of 500-12000 tokens: 65 us
+  // with 2048 workgroups of a tile per wave, 59 us with 700 of four). Larger batches get about 2048 workgroups, whose
+  // uneven progress then averages out (one round took 0.69 against 0.45 ms at 32 x 32768 tokens).
+  const uint64_t tiles_all = tile_work * sh.kv_heads;
   const uint32_t tps = static_cast<uint32_t>(
-      std::clamp<uint64_t>((tile_work * sh.kv_heads + 2047u) / 2048u, 4u, 256u));
+      tiles_all <= 512u * 32u ? std::max<uint64_t>((tiles_all + 511u) / 512u, 4u)
+                              : std::clamp<uint64_t>((tiles_all + 2047u) / 2048u, 32u, 256u));
 
   std::vector<AttnItem> items(reqs.size());
   uint64_t floats = 0;
@@ -625,7 +634,12 @@ hipError_t AttnRunner::run(const std::vector<AttnRequest> &reqs, const AttnShape
     it.window = r.window;
     it.scale_log2 = r.softmax_scale * 1.4426950408889634f;
     it.flags = r.flags;
-    it.asplits = (it.active_count + kActiveTokens - 1u) / kActiveTokens;
+    if (it.mfma_nb) {  // the MFMA kernel's last split takes the active page along
+      if (it.active_count) it.page_splits = std::max(it.page_splits, 1u);
+      it.asplits = 0u;
+    } else {
+      it.asplits = (it.active_count + kActiveTokens - 1u) / kActiveTokens;
+    }
     it.nsplit = (it.mfma_nb ? it.page_splits : 0u) + it.vsplits + it.asplits;
     if (it.nsplit == 0u) it.nsplit = 1u;  // nothing visible: one empty split, the row comes out 0
     it.ws_offset = floats;
@@ -638,7 +652,7 @@ hipError_t AttnRunner::run(const std::vector<AttnRequest> &reqs, const AttnShape
     error = "attention batch exceeds the launch grid (too many query tokens or items in one call)";
     return hipErrorInvalidValue;
   }
-  // the launches' work lists (prefix sums of their items' workgroups), uploaded behind the items: the VALU kernel's,
+  // the launches' work lists (prefix sums of their items' units), uploaded behind the items: the VALU kernel's,
   // the merge's, then one per MFMA mode in use
   const size_t n = items.size();
   std::vector<uint32_t> modes;
@@ -665,7 +679,7 @@ hipError_t AttnRunner::run(const std::vector<AttnRequest> &reqs, const AttnShape
       else if (l == 1)
         at += uint64_t(it.q_tokens) * sh.q_heads;
       else if (it.mfma_nb == modes[l - 2])
-        at += nib_mfma_workgroups(it, sh);
+        at += nib_mfma_units(it, sh);
     }
     totals[l] = static_cast<uint32_t>(at);
   }
@@ -695,7 +709,7 @@ hipError_t AttnRunner::run(const std::vector<AttnRequest> &reqs, const AttnShape
   const uint32_t *d_lists = reinterpret_cast<const uint32_t *>(static_cast<const char *>(ws_) + list_at);
   auto work = [&](size_t l) { return WorkList{d_lists + l * (n + 1), static_cast<uint32_t>(n), totals[l]}; };
   const dim3 block(hw * lg);
-  // the VALU kernel serves items without the MFMA path, every active page and every item with nothing visible
+  // the VALU kernel serves items without the MFMA path, the pages that path refuses and items with nothing visible
   if (totals[0]) switch (lg) {
     case 4: e = launch_attn_lg<4>(G, work(0), block, stream, d_items, sh, hw, hgroups, qchunks, partials); break;
     case 8: e = launch_attn_lg<8>(G, work(0), block, stream, d_items, sh, hw, hgroups, qchunks, partials); break;

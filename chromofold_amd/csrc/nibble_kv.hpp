@@ -59,14 +59,14 @@ struct AttnItem {
   const cf_device_page_descriptor *pages;
   uint32_t page_count;
   uint32_t units_per_split;  // pages (VALU kernel) or 64-token tiles (MFMA kernel) per context split
-  uint32_t page_splits;      // splits over the sealed pages
+  uint32_t page_splits;      // splits over the sealed pages (on the MFMA path the last one takes the active page along)
   uint32_t mfma_nb;          // 0: the VALU kernel reads the pages; 1/2/4: the MFMA kernel, scale blocks per row;
                              // kMfmaContract: the MFMA kernel reads the pages mfma_page_ok accepts (nibble_page.hpp)
   uint32_t vsplits;          // splits of the VALU kernel over the pages, after the MFMA kernel's page_splits (none
                              // for 1/2/4; for kMfmaContract they take only the pages the MFMA kernel refuses)
   uint32_t vunits;           // pages per VALU split (at most 64)
   uint32_t asplits;          // splits of the VALU kernel over the active page's tokens (kActiveTokens each), the last
-                             // of the item's nsplit
+                             // of the item's nsplit (none with mfma_nb)
   uint32_t mfma_cap;         // kMfmaContract: tokens a page may hold on the MFMA path (16 per planned chunk)
   const float *active_k;
   const float *active_v;
@@ -100,14 +100,15 @@ inline uint32_t mfma_sets(uint32_t head_dim, uint32_t block_size) {
 // a 64-token page at 8 partials for the merge.
 constexpr uint32_t kActiveTokens = 8u;
 
-// Workgroups of one launch: item i owns [first[i], first[i + 1]) (device array of items + 1; nibble_work.hpp).
+// Units of one launch: item i owns [first[i], first[i + 1]) (device array of items + 1; nibble_work.hpp). A unit is
+// a workgroup (VALU kernel), a wave (merge) or a workgroup per KV head (MFMA kernel).
 struct WorkList {
   const uint32_t *first;
   uint32_t items, total;
 };
 
-// Workgroups of the MFMA kernel for one item (page splits x query tokens x KV heads x chunks of 4 query heads).
-uint64_t nib_mfma_workgroups(const AttnItem &it, const AttnShape &sh);
+// Units of the MFMA kernel for one item (page splits x query tokens x chunks of 4 query heads).
+uint64_t nib_mfma_units(const AttnItem &it, const AttnShape &sh);
 
 // Launch of the MFMA kernel over the items whose mfma_nb == nb (the others own no workgroup of `work`).
 hipError_t launch_nib_mfma(uint32_t nb, const AttnItem *items, const WorkList &work, const AttnShape &sh, float *ws,
