@@ -1952,8 +1952,13 @@ uint32_t cu_count() {
 // Not for
 //   * a single sequence, which cannot be ragged: the splits' smaller workgroups start sooner (17.3 against 24 us at 2003
 //     tokens);
+//   * contexts that the splits leave with less than two chain pairs per wavefront: there is little to balance, and the
+//     span launch's longer prologue and its merge cost 5 us (20 x 2000 tokens: 27.8 against 32.4 us, 4 x 300: 13.8
+//     against 20.2);
 //   * the one-split wide shape from kSpanMaxPairs pairs per wavefront up: it needs no merge, and a batch padded to one
-//     length loses the merge and the longer prologue to a span launch (32 x 32768 tokens: 397 against 405 us);
+//     length loses the merge and the longer prologue to a span launch (32 x 32768 tokens: 397 against 405 us; at 32 x
+//     4096, 2.7 pairs per wavefront, 52.4 against 55.5 us padded to one length but 48.1 against 27.6 us ragged from 100
+//     tokens);
 //   * larger grids: one workgroup per unit, which the dispatcher balances and whose neighbours share a common prefix in
 //     L1;
 //   * callers who fix the splits, or whose workspace is too small for the span states.
@@ -1988,7 +1993,8 @@ BatchedPlan batched_plan(const cf_kv_batched_desc *d) {
   if (d->splits != 0 || d->seq_count < 2 || d->seq_count > kSpanMaxSeqs ||
       static_cast<uint64_t>(d->seq_count) * d->kv_head_count >= 3u * cu_count())
     return p;
-  if (p.waves == 12u && p.splits == 1u && (d->max_groups + 1) / 2 >= kSpanMaxPairs * kWavesWide) return p;
+  const uint32_t pairs = (d->max_groups + 1) / 2, lanes = p.splits * p.waves;  // wavefronts of the longest context
+  if (pairs < 2 * lanes || (p.waves == 12u && p.splits == 1u && pairs >= kSpanMaxPairs * lanes)) return p;
   return {1u, 12u, span_workgroups(d->kv_head_count)};
 }
 

@@ -11,7 +11,8 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
-RAGGED = [1, 64, 65, 128, 129, 3000, 16, 700, 191, 192, 193, 257]
+RAGGED = [1, 64, 65, 128, 129, 3100, 16, 700, 191, 192, 193, 257] + [1, 30, 64, 900, 5, 128, 1000, 2]
+MANY = [7, 64, 100, 65] * 34 + [3100, 1, 129, 64]
 
 
 def _reference(q, k, v, tokens, scale):
@@ -31,14 +32,14 @@ def _reference(q, k, v, tokens, scale):
 
 
 @pytest.mark.parametrize("codec,H,gqa,D,lens,raw", [
-    ("rans", 8, 4, 128, RAGGED, None),
-    ("rans", 2, 3, 128, [5000, 40, 1], None),              # one sequence over most workgroups
-    ("rans", 1, 1, 64, [100, 9000, 90, 64], None),         # one KV head: a workgroup per CU for it
-    ("rans", 4, 2, 64, RAGGED[::-1], None),
-    ("rans", 3, 4, 128, [512] * 7, None),                  # all alike, no divisor of anything
-    ("rans", 8, 4, 128, [300, 700, 500], {0: 2, 1: 3, 2: 8}),  # raw groups, odd and whole sequences
-    ("int8", 4, 2, 64, RAGGED, None),
-    ("int8", 8, 4, 128, [2000, 1, 900, 63], None),
+    ("rans", 8, 4, 128, RAGGED, None),                      # one long sequence over many workgroups
+    ("rans", 1, 1, 64, MANY, None),                         # one KV head: every CU's workgroup on it
+    ("rans", 7, 3, 64, RAGGED[::-1], None),
+    ("rans", 16, 2, 64, [1024] * 25, None),                 # all alike, no divisor of anything
+    ("rans", 8, 4, 128, ([1100, 3, 70] * 17)[:50], None),   # more units than CUs
+    ("rans", 8, 4, 128, RAGGED, {0: 1, 1: 1, 5: 9, 7: 3, 15: 15}),  # raw groups, odd counts and whole sequences
+    ("int8", 8, 2, 64, RAGGED, None),
+    ("int8", 8, 4, 128, RAGGED[::-1], None),
 ])
 @pytest.mark.parametrize("hide", [(), (0, 1), (-1,)])
 def test_spans_match_the_split_launch(codec, H, gqa, D, lens, raw, hide):
@@ -67,6 +68,7 @@ def test_spans_match_the_split_launch(codec, H, gqa, D, lens, raw, hide):
     kvb.seq_tokens = torch.from_numpy(tok.astype(np.int32)).to(dev)
     qd, pd = torch.from_numpy(q).to(dev), torch.from_numpy(pos.astype(np.int32)).to(dev)
     scale = 1.0 / np.sqrt(D)
+    assert kvb.desc(qd, qd, pd, scale).workspace_bytes > 0, "one split and no span launch"
     outs = []
     for splits in (0, 1):
         out = torch.full(q.shape, float("nan"), device=dev)
@@ -98,9 +100,9 @@ def test_span_in_a_graph_and_with_a_small_workspace():
     from chromofold_amd import kv
     dev = torch.device("cuda:0")
     rng = np.random.default_rng(5)
-    H, gqa, D, lens = 4, 4, 128, [900, 70, 2000, 333]
+    H, gqa, D, lens = 8, 4, 128, RAGGED
     data = [tuple(rng.standard_normal((H, T, D)).astype(np.float32) for _ in range(2)) for T in lens]
-    tables = np.concatenate([kv.build_table(x[h][:64].reshape(-1, 16, D)) for h in range(H) for x in data[0]])
+    tables = np.concatenate([kv.build_table(x[h][:64].reshape(-1, 16, D)) for h in range(H) for x in data[5]])
     kvb = kv.build_batched(kv.CODEC_RANS_HYBRID, lambda s: data[s], len(lens), H, np.array(lens), D, tables, dev,
                            encoder="device")
     q = torch.from_numpy(rng.standard_normal((len(lens), H * gqa, D)).astype(np.float32)).to(dev)
@@ -117,7 +119,7 @@ def test_span_in_a_graph_and_with_a_small_workspace():
         run()
     full = kvb.seq_tokens.clone()
     for i in range(4):
-        kvb.seq_tokens.copy_(torch.tensor([5, 1000 + i, 64, 0], device=dev))
+        kvb.seq_tokens.copy_(torch.minimum(full, torch.arange(len(lens), device=dev) * (40 + i)))
         run()
         kvb.seq_tokens.copy_(full)
         out.fill_(float("nan"))
