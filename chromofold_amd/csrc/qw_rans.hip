@@ -22,6 +22,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <utility>
 
 #include "cf_device.hpp"
 #include "chromofold/chromofold_qw.h"
@@ -29,17 +30,17 @@
 
 namespace {
 
-typedef short bf16x4_t __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
 constexpr int kThreads = 1024;
 constexpr int kWaves = kThreads / 64;
-constexpr int kPer = CF_QW_CHUNK_STRIPES / kWaves;           // stripes per wave per chunk, decoded together
 constexpr int kSlots = 1 << CF_QW_RANS_PROB_BITS;           // 4096 table entries
 constexpr int kSlotW16 = CF_QW_MAX_CHUNK_WORDS;              // largest chunk slot, 16-bit words
 constexpr int kMaxTiles = 4;
 
-static_assert(kPer * kWaves == CF_QW_CHUNK_STRIPES, "the chunk's stripes split evenly over the waves");
+static_assert(kWaves == CF_QW_CHUNK_STRIPES, "one stripe of a chunk per wave");
 static_assert(kSlotW16 <= 4 * kThreads * 8, "four 16-byte staging loads per thread cover the largest slot");
 static_assert(CF_QW_STRIPE_COLS == 256 && CF_QW_BAND_ROWS == 16, "the lane / column map of chromofold_qw.h");
 
@@ -113,10 +114,6 @@ __device__ __forceinline__ uint4 x_frag8(const uint16_t *__restrict__ x, int b, 
   return make_uint4(v[0] | (v[1] << 16), v[2] | (v[3] << 16), v[4] | (v[5] << 16), v[6] | (v[7] << 16));
 }
 
-__device__ __forceinline__ bf16x4_t as_bf16x4(uint32_t a, uint32_t b) {  // {a.lo, a.hi, b.lo, b.hi}
-  return __builtin_bit_cast(bf16x4_t, make_uint2(a, b));
-}
-
 // One decode step of a lane: returns the pair's two weights (bf16 x2); x and the wave's cursor advance.
 __device__ __forceinline__ uint32_t rans_step(const uint2 *__restrict__ tab, uint32_t &x,
                                               const uint16_t *__restrict__ &cur) {
@@ -134,22 +131,31 @@ __device__ __forceinline__ uint32_t rans_step(const uint2 *__restrict__ tab, uin
   return e.y;
 }
 
-template <int NT, bool FAST, int SL, int XR>
-__global__ void __launch_bounds__(kThreads) qw_rans_kernel(RansArgs a) {
+// NT: batch tiles of 16 rows. FAST: whole stripes, aligned x, 32-bit offsets (launch_rans). SL: 16-byte staging loads per
+// thread and chunk. XR: x rows staged in LDS. PIPE: several chunks, each chunk's slot, states, offsets and scales loaded
+// while the one before it is decoded (one chunk after another cost a memory latency and a table build each: 14 us a
+// chunk at 48 rows of 14336 columns); a single chunk needs no such registers, so that two workgroups fit a CU.
+template <int NT, bool FAST, int SL, int XR, bool PIPE>
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(FAST && NT == 1 && SL == 2 ? 8 : 4)))
+qw_rans_kernel(RansArgs a) {
   static_assert(kThreads == 1024 && (SL == 2 || SL == 4), "staging loads per thread");
+  // four batch tiles leave no registers for the next chunk (spills: 55 against 52 us at 64 x 9216 columns)
+  constexpr bool AHEAD = PIPE && NT < 4;
   static_assert(XR == 0 || (NT == 1 && FAST), "x rows staged in LDS: one batch tile, whole stripes");
-  __shared__ __attribute__((aligned(16))) uint2 s_tab[kSlots];
-  // the chunk slot; reused by the reduction. A stripe's cursor starts at most at the slot's end (clamped) and a step
-  // moves it by at most 64, with reads up to 63 words past it: 32 steps stay within kSlotW16 + 64 * 33 words
-  // whatever the stream holds.
-  __shared__ __attribute__((aligned(16))) uint16_t s_slot[kSlotW16 + 64 * 33];
+  // The table, then the chunk slot; both reused by the reduction. A stripe's cursor starts at most at the slot's end
+  // (clamped) and a step moves it by at most 64, with reads up to 63 words past it: 32 steps stay within the slot and
+  // 64 * 33 words whatever the stream holds.
+  constexpr int kTabBytes = kSlots * 8, kSlotBytes = (SL * kThreads * 8 + 64 * 33) * 2;
+  __shared__ __attribute__((aligned(16))) uint8_t s_mem[kTabBytes + kSlotBytes];
+  uint2 *s_tab = reinterpret_cast<uint2 *>(s_mem);
+  uint16_t *s_slot = reinterpret_cast<uint16_t *>(s_mem + kTabBytes);
   __shared__ __attribute__((aligned(16))) uint32_t s_cum[260];
   // XR > 0 (a batch of at most XR rows): the chunk's x columns of rows 0..XR-1, staged once per workgroup (8 bytes
   // per thread and row) instead of every lane loading its 16-byte fragments from global memory, where the 16 row
   // lanes of a lane group would all fetch the same row (B = 1: 9.2 -> 8.8 us per call)
   constexpr int kXCols = CF_QW_CHUNK_STRIPES * CF_QW_STRIPE_COLS;
   __shared__ __attribute__((aligned(16))) uint16_t s_x[XR > 0 ? XR * kXCols : 8];
-  static_assert(sizeof(s_slot) >= kWaves * NT * 256 * 4, "reduction fits the slot buffer");
+  static_assert(sizeof(s_mem) >= kWaves * NT * 256 * 4, "reduction fits the table and slot buffers");
 
   const int t = threadIdx.x, lane = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);  // in a scalar register: stripe choices are wave-uniform
@@ -164,164 +170,178 @@ __global__ void __launch_bounds__(kThreads) qw_rans_kernel(RansArgs a) {
   for (int i = 0; i < NT; ++i) acc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
   const size_t band_words = static_cast<size_t>(a.nchunks - 1) * a.chunk_words + a.last_words;
-  for (int ch = 0; ch < a.nchunks; ++ch) {
-    const int slot_words = ch + 1 == a.nchunks ? a.last_words : a.chunk_words;
-    const int n16 = slot_words / 8;  // 16-byte units of the slot
-    // the wave's stripes: wave and wave + kWaves of the chunk (wave-uniform)
-    int st[kPer];
-    bool active[kPer];
-#pragma unroll
-    for (int c = 0; c < kPer; ++c) {
-      const int stripe = ch * CF_QW_CHUNK_STRIPES + wave + kWaves * c;
-      active[c] = stripe < a.nstripes;
-      st[c] = min(stripe, a.nstripes - 1);
-    }
-    // ---- straight-line loads (no branch, no select on a loaded value: either would make the compiler wait for
-    // the loads issued before): the band's cumulative starts (first used by the table build; every wave loads
-    // them, wave 0 uses them), the slot, the lanes' states, the stripe offsets, scales, first x fragments
-    const uint2 cw = reinterpret_cast<const uint2 *>(a.cums + static_cast<size_t>(band) * 256)[lane];
-    asm volatile("" ::: "memory");  // issued first: not sunk into the table build, behind the other loads
-    const uint4 *slot = a.words + (band * band_words + static_cast<size_t>(ch) * a.chunk_words) / 8;
-    // SL unconditional 16-byte loads per thread (clamped addresses: a branch around a load makes the compiler wait
-    // for the loads before it) into named registers (a private array here is promoted to LDS and stored there at
-    // once); the host picks SL = 2 when the slot fits 2048 16-byte units. (Letting only the first four wavefronts
-    // load the whole slot, so that it is in flight earlier, measured slower: their longer prologues delay the
-    // table barrier.)
-    const uint32_t last = static_cast<uint32_t>(n16 - 1), tt = static_cast<uint32_t>(t);
-    const uint4 st0 = slot[min(tt, last)], st1 = slot[min(tt + kThreads, last)];
-    uint4 st2 = make_uint4(0, 0, 0, 0), st3 = st2;
+  // What a chunk needs beside x: its slot (SL unconditional 16-byte loads per thread with clamped addresses: a branch
+  // around a load, or a select on a loaded value, makes the compiler wait for the loads before it; named vector members:
+  // arrays, and uint4 members, end up in LDS or scratch, stored there at once), the lane's state, the stripe's offset, the scales.
+  struct Chunk {
+    u32x4_t st0, st1, st2, st3;
+    uint32_t x, soff;
+    float sc0, sc1, sc2, sc3;
+  };
+  auto slot_units = [&](int ch) { return (ch + 1 == a.nchunks ? a.last_words : a.chunk_words) / 8; };
+  auto stripe_of = [&](int ch) { return min(ch * CF_QW_CHUNK_STRIPES + wave, a.nstripes - 1); };
+  auto load_chunk = [&](int ch, Chunk &c) {
+    const u32x4_t *slot = reinterpret_cast<const u32x4_t *>(a.words) +
+                          (band * band_words + static_cast<size_t>(ch) * a.chunk_words) / 8;
+    const uint32_t last = static_cast<uint32_t>(slot_units(ch) - 1), tt = static_cast<uint32_t>(t);
+    c.st0 = slot[min(tt, last)];
+    c.st1 = slot[min(tt + kThreads, last)];
     if constexpr (SL == 4) {
-      st2 = slot[min(tt + 2 * kThreads, last)];
-      st3 = slot[min(tt + 3 * kThreads, last)];
+      c.st2 = slot[min(tt + 2 * kThreads, last)];
+      c.st3 = slot[min(tt + 3 * kThreads, last)];
     }
-    uint32_t x[kPer], soff[kPer];
-    float sc[kPer][4];
-#pragma unroll
-    for (int c = 0; c < kPer; ++c) {
-      x[c] = a.states[(static_cast<size_t>(band) * a.nstripes + st[c]) * 64 + lane];
-      soff[c] = min(a.offsets[static_cast<size_t>(band) * a.nstripes + st[c]], static_cast<uint32_t>(slot_words));
-    }
-    // x fragments by half segment (8 columns of each lane group; half h = 2 q + (j >> 1)) in a ring of XH: one tile
-    // holds all 8 halves of both stripes, more tiles prefetch XH - 1 halves ahead of the decode (register budget)
-    constexpr int XH = NT == 1 ? 8 : NT == 2 ? 4 : 2;
-    uint4 xf[kPer][XH][NT];
-    // FAST: 32-bit per-lane offsets from wave-uniform bases (the prologue's address arithmetic is a large part of
-    // its issue time, which the wavefronts of a SIMD spend one after another before the first barrier)
-    const uint16_t *xb = a.x + static_cast<size_t>(a.bt0) * 16 * K;  // wave-uniform
-    uint32_t xoff[NT];
-    if constexpr (FAST) {
-#pragma unroll
-      for (int c = 0; c < kPer; ++c) {  // 4 scales of the lane's row in one 16-byte load (nseg: a multiple of 4)
-        const float4 s4 = *reinterpret_cast<const float4 *>(
-            a.scales + 4 * st[c] + static_cast<uint32_t>(row) * static_cast<uint32_t>(nseg));
-        sc[c][0] = s4.x;
-        sc[c][1] = s4.y;
-        sc[c][2] = s4.z;
-        sc[c][3] = s4.w;
-      }
-#pragma unroll
-      for (int i = 0; i < NT; ++i) {  // rows past the batch read the batch's last row (outputs never written)
-        const uint32_t rr = static_cast<uint32_t>(min((a.bt0 + i) * 16 + r, B - 1) - a.bt0 * 16);
-        xoff[i] = rr * static_cast<uint32_t>(K) + static_cast<uint32_t>(16 * g);
-      }
+    const int st = stripe_of(ch);
+    c.x = a.states[(static_cast<size_t>(band) * a.nstripes + st) * 64 + lane];
+    c.soff = min(a.offsets[static_cast<size_t>(band) * a.nstripes + st], static_cast<uint32_t>(8 * slot_units(ch)));
+    if constexpr (FAST) {  // 4 scales of the lane's row in one 16-byte load (nseg: a multiple of 4)
+      const float4 s4 = *reinterpret_cast<const float4 *>(
+          a.scales + 4 * st + static_cast<uint32_t>(row) * static_cast<uint32_t>(nseg));
+      c.sc0 = s4.x;
+      c.sc1 = s4.y;
+      c.sc2 = s4.z;
+      c.sc3 = s4.w;
     } else {
-#pragma unroll
-      for (int c = 0; c < kPer; ++c)
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-          sc[c][q] = a.scales[static_cast<size_t>(row) * nseg + min(4 * st[c] + q, nseg - 1)];
+      const float *s4 = a.scales + static_cast<size_t>(row) * nseg;
+      c.sc0 = s4[min(4 * st, nseg - 1)];
+      c.sc1 = s4[min(4 * st + 1, nseg - 1)];
+      c.sc2 = s4[min(4 * st + 2, nseg - 1)];
+      c.sc3 = s4[min(4 * st + 3, nseg - 1)];
     }
-    auto load_x = [&](int h) {
-#pragma unroll
-      for (int c = 0; c < kPer; ++c)
-#pragma unroll
-        for (int i = 0; i < NT; ++i) {
-          const int col = st[c] * 256 + 64 * (h >> 1) + 8 * (h & 1);
-          if constexpr (XR > 0)
-            xf[c][h % XH][i] = *reinterpret_cast<const uint4 *>(
-                s_x + min(r, XR - 1) * kXCols + (col - ch * kXCols) + 16 * g);
-          else if constexpr (FAST)
-            xf[c][h % XH][i] = *reinterpret_cast<const uint4 *>(xb + xoff[i] + col);
-          else
-            xf[c][h % XH][i] = x_frag8(a.x, (a.bt0 + i) * 16 + r, B, col + 16 * g, K);
-        }
-    };
-    uint2 xs[XR > 0 ? XR : 1];
-    if constexpr (XR > 0) {  // x rows 0..XR-1 (rows past the batch repeat its last row), 4 columns per thread
-      const int c4 = min(ch * kXCols + 4 * t, K - 4);
-#pragma unroll
-      for (int rr = 0; rr < XR; ++rr)
-        xs[rr] = *reinterpret_cast<const uint2 *>(xb + static_cast<uint32_t>(min(rr, B - 1)) * static_cast<uint32_t>(K) + c4);
-    } else {
-#pragma unroll
-      for (int h = 0; h < XH - 1; ++h) load_x(h);
-    }
-    // ---- the band's table while the loads are in flight (rebuilt for every chunk: a build under a branch would
-    // let the compiler sink the table load into it, behind the others)
-    build_table(cw, a.zero, s_tab, s_cum);
-    uint4 *s_slot4 = reinterpret_cast<uint4 *>(s_slot);
-    const uint32_t n = static_cast<uint32_t>(n16);
-    if (tt < n) s_slot4[tt] = st0;
-    if (tt + kThreads < n) s_slot4[tt + kThreads] = st1;
+  };
+  auto store_chunk = [&](int ch, const Chunk &c) {
+    u32x4_t *s_slot4 = reinterpret_cast<u32x4_t *>(s_slot);
+    const uint32_t n = static_cast<uint32_t>(slot_units(ch)), tt = static_cast<uint32_t>(t);
+    if (tt < n) s_slot4[tt] = c.st0;
+    if (tt + kThreads < n) s_slot4[tt + kThreads] = c.st1;
     if constexpr (SL == 4) {
-      if (tt + 2 * kThreads < n) s_slot4[tt + 2 * kThreads] = st2;
-      if (tt + 3 * kThreads < n) s_slot4[tt + 3 * kThreads] = st3;
+      if (tt + 2 * kThreads < n) s_slot4[tt + 2 * kThreads] = c.st2;
+      if (tt + 3 * kThreads < n) s_slot4[tt + 3 * kThreads] = c.st3;
     }
+  };
+
+  // x fragments in units of XU halves of a 64-column segment (8 columns of each lane group), XS units in a ring, XS - 1
+  // ahead of the decode, across chunks too. Both halves of a segment together where registers allow: they share the row's
+  // 128-byte line, which the other wavefronts' rows push out of L1 before a later load.
+  constexpr int XU = NT == 4 && PIPE ? 1 : 2;
+  constexpr int XS = NT == 1 && FAST ? 4 : FAST ? 2 : 1;
+  uint4 xf[XU * XS][NT];
+  // FAST: 32-bit per-lane offsets from wave-uniform bases (the prologue's address arithmetic is a large part of
+  // its issue time, which the wavefronts of a SIMD spend one after another before the first barrier)
+  const uint16_t *xb = a.x + static_cast<size_t>(a.bt0) * 16 * K;  // wave-uniform
+  uint32_t xoff[NT];
+  if constexpr (FAST) {
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {  // rows past the batch read the batch's last row (outputs never written)
+      const uint32_t rr = static_cast<uint32_t>(min((a.bt0 + i) * 16 + r, B - 1) - a.bt0 * 16);
+      xoff[i] = rr * static_cast<uint32_t>(K) + static_cast<uint32_t>(16 * g);
+    }
+  }
+  auto load_x = [&](int st, auto uc) {  // unit uc of stripe st
+    constexpr int u = decltype(uc)::value;
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+      for (int hh = 0; hh < XU; ++hh) {
+        const int h = XU * u + hh, col = st * 256 + 64 * (h >> 1) + 8 * (h & 1);
+        uint4 &f = xf[XU * (u % XS) + hh][i];
+        if constexpr (XR > 0)
+          f = *reinterpret_cast<const uint4 *>(s_x + min(r, XR - 1) * kXCols + col % kXCols + 16 * g);
+        else if constexpr (FAST)
+          f = *reinterpret_cast<const uint4 *>(xb + xoff[i] + col);
+        else
+          f = x_frag8(a.x, (a.bt0 + i) * 16 + r, B, col + 16 * g, K);
+      }
+  };
+  auto load_x_first = [&](int st) {
+    [&]<int... Q>(std::integer_sequence<int, Q...>) {
+      (load_x(st, std::integral_constant<int, Q>{}), ...);
+    }(std::make_integer_sequence<int, XS - 1>{});
+  };
+  auto stage_x = [&](int ch, uint2 (&xs)[XR > 0 ? XR : 1]) {  // rows past the batch repeat its last row
+    const int c4 = min(ch * kXCols + 4 * t, K - 4);
+#pragma unroll
+    for (int rr = 0; rr < XR; ++rr)
+      xs[rr] = *reinterpret_cast<const uint2 *>(xb + static_cast<uint32_t>(min(rr, B - 1)) * static_cast<uint32_t>(K) + c4);
+  };
+
+  // ---- the band's cumulative starts are issued first (not sunk into the table build, behind the other loads); the
+  // table is built while the first chunk's loads are in flight
+  const uint2 cw = reinterpret_cast<const uint2 *>(a.cums + static_cast<size_t>(band) * 256)[lane];
+  asm volatile("" ::: "memory");
+  Chunk cur;
+  load_chunk(0, cur);
+  uint2 xs[XR > 0 ? XR : 1];
+  if constexpr (XR > 0) stage_x(0, xs);
+  else load_x_first(stripe_of(0));
+  build_table(cw, a.zero, s_tab, s_cum);
+
+  for (int ch = 0; ch < (PIPE ? a.nchunks : 1); ++ch) {
+    const int st = stripe_of(ch);
+    const bool active = ch * CF_QW_CHUNK_STRIPES + wave < a.nstripes;
+    if constexpr (PIPE && !AHEAD) {
+      if (ch > 0) {
+        load_chunk(ch, cur);
+        load_x_first(st);
+      }
+    }
+    store_chunk(ch, cur);
     if constexpr (XR > 0) {
 #pragma unroll
       for (int rr = 0; rr < XR; ++rr) *reinterpret_cast<uint2 *>(s_x + rr * kXCols + 4 * t) = xs[rr];
     }
-    __syncthreads();
-    if constexpr (XR > 0) {
-#pragma unroll
-      for (int h = 0; h < XH - 1; ++h) load_x(h);
+    uint32_t x = cur.x;
+    const uint16_t *cp = s_slot + __builtin_amdgcn_readfirstlane(cur.soff);  // scalar cursor
+    const float sc[4] = {cur.sc0, cur.sc1, cur.sc2, cur.sc3};
+    if constexpr (PIPE) lds_barrier();  // (the x loads in flight are not waited for)
+    else __syncthreads();
+    const int stn = AHEAD ? stripe_of(min(ch + 1, a.nchunks - 1)) : 0;
+    if constexpr (AHEAD) {  // the last chunk loads itself again
+      load_chunk(min(ch + 1, a.nchunks - 1), cur);
+      if constexpr (XR > 0) stage_x(min(ch + 1, a.nchunks - 1), xs);
     }
-    // ---- decode + MFMA: the wave's two stripes step together (two independent chains); a stripe past the
-    // matrix (last chunk) decodes the matrix's last stripe again and its partials are dropped
-    const uint16_t *cur[kPer];
+    if constexpr (XR > 0) load_x_first(st);
+    // ---- decode + MFMA: four steps are 8 columns of each lane group, the k = 32 of one MFMA; a stripe past the matrix
+    // (last chunk) decodes the matrix's last stripe again and its partials are dropped
+    f32x4_t part[NT];
+    [&]<int... H>(std::integer_sequence<int, H...>) {
+      (
+          [&] {
+            constexpr int h = H, q = H / 2, units = 8 / XU, ahead = h / XU + XS - 1;
+            if constexpr (h % XU == 0) {
+              if constexpr (ahead < units) load_x(st, std::integral_constant<int, ahead>{});
+              else if constexpr (AHEAD && XR == 0) load_x(stn, std::integral_constant<int, ahead - units>{});
+            }
+            if constexpr (h % 2 == 0) {
 #pragma unroll
-    for (int c = 0; c < kPer; ++c) cur[c] = s_slot + __builtin_amdgcn_readfirstlane(soff[c]);  // scalar cursor
+              for (int i = 0; i < NT; ++i) part[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+            }
+            uint4 w;
+            w.x = rans_step(s_tab, x, cp);
+            w.y = rans_step(s_tab, x, cp);
+            w.z = rans_step(s_tab, x, cp);
+            w.w = rans_step(s_tab, x, cp);
+            const bf16x8_t bfrag = __builtin_bit_cast(bf16x8_t, w);
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      f32x4_t part[kPer][NT];
+            for (int i = 0; i < NT; ++i)
+              part[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, xf[XU * (h / XU % XS) + h % XU][i]), bfrag, part[i],
+                                                               0, 0, 0);
+            if constexpr (h % 2 == 1) {
+              if (active) {  // wave-uniform
 #pragma unroll
-      for (int c = 0; c < kPer; ++c)
+                for (int i = 0; i < NT; ++i)
 #pragma unroll
-        for (int i = 0; i < NT; ++i) part[c][i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int h = 2 * q + (j >> 1);
-        if ((j & 1) == 0 && h + XH - 1 < 8) load_x(h + XH - 1);
-        uint32_t w0[kPer], w1[kPer];
-#pragma unroll
-        for (int c = 0; c < kPer; ++c) w0[c] = rans_step(s_tab, x[c], cur[c]);
-#pragma unroll
-        for (int c = 0; c < kPer; ++c) w1[c] = rans_step(s_tab, x[c], cur[c]);
-#pragma unroll
-        for (int c = 0; c < kPer; ++c) {
-          const bf16x4_t bfrag = as_bf16x4(w0[c], w1[c]);
-#pragma unroll
-          for (int i = 0; i < NT; ++i) {
-            const uint4 &u = xf[c][h % XH][i];
-            const bf16x4_t afrag = (j & 1) ? as_bf16x4(u.z, u.w) : as_bf16x4(u.x, u.y);
-            part[c][i] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(afrag, bfrag, part[c][i], 0, 0, 0);
-          }
-        }
-      }
-#pragma unroll
-      for (int c = 0; c < kPer; ++c) {
-        if (!active[c]) continue;  // wave-uniform
-#pragma unroll
-        for (int i = 0; i < NT; ++i)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) acc[i][e] += sc[c][q] * part[c][i][e];  // the lane's output column is row r
-      }
-    }
-    __syncthreads();  // slot buffer free for the next chunk (or the reduction)
+                  for (int e = 0; e < 4; ++e) acc[i][e] += sc[q] * part[i][e];  // the lane's output column is row r
+              }
+            }
+          }(),
+          ...);
+    }(std::make_integer_sequence<int, 8>{});
+    if constexpr (PIPE) lds_barrier();  // slot buffer free for the next chunk (or the reduction)
+    else __syncthreads();
   }
 
   // ---- fixed-order cross-wave reduction, one write of y per (b, m)
-  float *red = reinterpret_cast<float *>(s_slot);
+  float *red = reinterpret_cast<float *>(s_mem);
 #pragma unroll
   for (int i = 0; i < NT; ++i)
 #pragma unroll
@@ -344,12 +364,34 @@ __global__ void __launch_bounds__(kThreads) qw_rans_kernel(RansArgs a) {
   }
 }
 
-template <int NT, bool FAST, int XR>
+uint32_t cu_count() {  // multiprocessors of the current device, per host thread
+  static thread_local int cached_dev = -1;
+  static thread_local uint32_t cached = 0;
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return 256;
+  if (dev != cached_dev) {
+    int cus = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
+    cached = static_cast<uint32_t>(cus);
+    cached_dev = dev;
+  }
+  return cached;
+}
+
+template <int NT, bool FAST, int XR, bool PIPE>
 void launch_rans_sl(const RansArgs &a, unsigned grid, hipStream_t s) {
+  // Two workgroups fit a CU in some variants. A grid of at most one per CU gets LDS that keeps them apart: the
+  // dispatcher otherwise puts pairs of them on one CU while others idle (4096 x 4096, one row: 9.6 against 8.2 us).
+  const unsigned apart = grid <= cu_count() ? 20480u : 0u;
   if (max(a.chunk_words, a.last_words) <= 2 * kThreads * 8)
-    qw_rans_kernel<NT, FAST, 2, XR><<<grid, kThreads, 0, s>>>(a);
+    qw_rans_kernel<NT, FAST, 2, XR, PIPE><<<grid, kThreads, apart, s>>>(a);
   else
-    qw_rans_kernel<NT, FAST, 4, XR><<<grid, kThreads, 0, s>>>(a);
+    qw_rans_kernel<NT, FAST, 4, XR, PIPE><<<grid, kThreads, apart, s>>>(a);
+}
+template <int NT, bool FAST, int XR>
+void launch_rans_pipe(const RansArgs &a, unsigned grid, hipStream_t s) {
+  if (a.nchunks > 1) launch_rans_sl<NT, FAST, XR, true>(a, grid, s);
+  else launch_rans_sl<NT, FAST, XR, false>(a, grid, s);
 }
 
 template <int NT>
@@ -361,11 +403,11 @@ void launch_rans(const RansArgs &a, unsigned grid, hipStream_t s) {
   // a batch of one row stages its x row in LDS (staging four rows for batches of up to four measured slower: 9.6
   // against 9.4 us at B = 4)
   if (fast && NT == 1 && a.B == 1)
-    launch_rans_sl<NT, true, NT == 1 ? 1 : 0>(a, grid, s);
+    launch_rans_pipe<NT, true, NT == 1 ? 1 : 0>(a, grid, s);
   else if (fast)
-    launch_rans_sl<NT, true, 0>(a, grid, s);
+    launch_rans_pipe<NT, true, 0>(a, grid, s);
   else
-    launch_rans_sl<NT, false, 0>(a, grid, s);
+    launch_rans_pipe<NT, false, 0>(a, grid, s);
 }
 
 }  // namespace
