@@ -96,7 +96,9 @@ __global__ void __launch_bounds__(256) table_prep_kernel(const uint8_t *__restri
   const uint32_t f = s < 0 ? 0u : (blob[2 * s] & 2047u);
   if (f == 0) atomicOr(&s_bad, 1u);
   atomicAdd(&s_total, f);
-  ctab[blockIdx.x * 256 + tid] = f | static_cast<uint32_t>(s < 0 ? 0 : s) << 16;
+  // {freq | cum << 16, floor(2^32 / freq)}: the coder's division (see rans_div)
+  reinterpret_cast<uint2 *>(ctab)[blockIdx.x * 256 + tid] =
+      make_uint2(f | static_cast<uint32_t>(s < 0 ? 0 : s) << 16, f <= 1 ? 0xFFFFFFFFu : static_cast<uint32_t>((1ull << 32) / f));
   __syncthreads();
   if (tid == 0) tvalid[blockIdx.x] = (!s_bad && s_total == 2048u) ? 1u : 0u;
 }
@@ -116,7 +118,9 @@ struct EncodeArgs {
   uint32_t *units, *status;
 };
 
-// Symbol word (4 symbols q + 128, symbol i in byte i) of lane (G, t), quad q, in the lane order of kv_codec_ext.h.
+// Symbol word (4 symbols, symbol i in byte i) of lane (G, t), quad q, in the lane order of kv_codec_ext.h. The RANS codec
+// keeps symbols as sign-magnitude bytes (sign << 7 | magnitude; 0x80, a negative zero, stands for -128), the form its raw
+// words and big bits are cut from with masks; the INT8 codec keeps q + 128.
 __device__ __forceinline__ uint32_t k_word(const uint32_t *kS, int G, int t, int q) {
   return kS[(G * 16 + t) * kKStride + q];
 }
@@ -124,22 +128,82 @@ __device__ __forceinline__ uint32_t v_word(const uint32_t *vT, int G, int t, int
   return vT[(G * kMaxDim + t + 16 * (q % ng)) * kVStride + q / ng];
 }
 
-// big bits (|q| >= 64: symbol >= 192 or <= 64) of the 4 symbols of a word, bit i for symbol i
-__device__ __forceinline__ uint32_t bigs_of(uint32_t w) {
-  uint32_t j = 0;
+// big bits (magnitude >= 64) of the 4 sign-magnitude symbols of a word, bit i for symbol i: bits 6, 14, 22, 30 brought
+// to bits 28..31 by one multiplication whose other partial products neither reach nor carry into them
+__device__ __forceinline__ uint32_t bigs_of(uint32_t w) { return (((w >> 6) & 0x01010101u) * 0x10204080u) >> 28; }
+
+// the offset-binary symbols q + 128 of a sign-magnitude word
+__device__ __forceinline__ uint32_t offset_binary(uint32_t w) {
+  uint32_t r = 0;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const uint32_t b = (w >> (8 * i)) & 255u;
-    j |= (b >= 192u || b <= 64u ? 1u : 0u) << i;
+    r |= (b == 128u ? 0u : b > 128u ? 256u - b : 128u + b) << (8 * i);
   }
-  return j;
+  return r;
 }
 
+// Four values of a page as a symbol word. The quotients are x * (1 / scale); where that may round to another integer
+// than the IEEE quotient x / scale (its error is below 3e-5 at quotients up to 128, so only within that distance of a
+// half), or is no number, the wavefront takes the exact division for the word (1.5 % of words). `exact` (wave-uniform):
+// the scale is so small or large that its reciprocal is not accurate.
+__device__ __forceinline__ uint32_t quant_word(const float (&x)[4], float scale, float rscale, bool exact, bool rans) {
+  float r[4];
+  bool doubt = exact;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float t = x[i] * rscale;
+    r[i] = __builtin_rintf(t);
+    doubt |= !(__builtin_fabsf(t - r[i]) < 0.5f - 3e-5f);  // also for NaN and infinities
+  }
+  uint32_t w;
+  if (__ballot(doubt) == 0) {
+    uint32_t mag = 0;
+    mag = __builtin_amdgcn_cvt_pk_u8_f32(__builtin_fabsf(r[0]), 0, mag);
+    mag = __builtin_amdgcn_cvt_pk_u8_f32(__builtin_fabsf(r[1]), 1, mag);
+    mag = __builtin_amdgcn_cvt_pk_u8_f32(__builtin_fabsf(r[2]), 2, mag);
+    mag = __builtin_amdgcn_cvt_pk_u8_f32(__builtin_fabsf(r[3]), 3, mag);
+    const uint32_t t01 = __builtin_amdgcn_perm(__float_as_uint(r[1]), __float_as_uint(r[0]), 0x0c0c0703u);
+    const uint32_t t23 = __builtin_amdgcn_perm(__float_as_uint(r[3]), __float_as_uint(r[2]), 0x07030c0cu);
+    w = mag | ((t01 | t23) & (mag + 0x7F7F7F7Fu) & 0x80808080u);  // no sign on a zero (magnitudes are at most 127)
+    if (!rans) {  // q + 128 = 128 + magnitude, or 128 - magnitude where the sign is set
+      const uint32_t sg = w & 0x80808080u, one = sg >> 7, m = (sg - one) | sg;
+      w = ((mag ^ m) + one) ^ 0x80808080u;  // two's complement per byte (magnitude >= 1 there), then the offset
+    }
+    return w;
+  }
+  w = 0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t b = quant8(x[i], scale);
+    w |= (!rans ? b : b >= 128u ? b - 128u : b == 0u ? 128u : 256u - b) << (8 * i);
+  }
+  return w;
+}
+// whether a sign-magnitude / offset-binary word holds a -128
+__device__ __forceinline__ bool has_minus128(uint32_t w, bool rans) {
+  const uint32_t z = rans ? w ^ 0x80808080u : w;  // a zero byte
+  return ((z - 0x01010101u) & ~z & 0x80808080u) != 0u;
+}
+
+// q = x / f, r = x % f for 1 <= f < 2^11 from m = floor(2^32 / f) (all ones for f = 1): mulhi(x, m) is the quotient or
+// one less (x (2^32 / f - m) < 2^32 for every 32-bit x)
+__device__ __forceinline__ void rans_div(uint32_t x, uint32_t f, uint32_t m, uint32_t &q, uint32_t &r) {
+  q = __umulhi(x, m);
+  r = x - q * f;
+  if (r >= f) {
+    ++q;
+    r -= f;
+  }
+}
+
+// DT: the head_dim (0: any), so that the index arithmetic of the usual ones is shifts.
+template <int DT>
 __global__ void __launch_bounds__(kEncThreads) encode_kernel(EncodeArgs a) {
   __shared__ uint32_t kS[2][4 * 16 * kKStride];
   __shared__ uint32_t vT[2][4 * kMaxDim * kVStride];
   __shared__ uint16_t s_words[2][2][kStreamCap];  // [stream][group of the unit]
-  __shared__ uint32_t s_tab[2][256];
+  __shared__ uint2 s_tab[2][256];
   __shared__ float s_scale[2][2][4];               // [group][K, V][page]
   __shared__ uint32_t s_tc[2][4], s_count[2][2], s_bad, s_minus[2];
 
@@ -151,7 +215,7 @@ __global__ void __launch_bounds__(kEncThreads) encode_kernel(EncodeArgs a) {
   const uint64_t half = (a.ngroups + 1) / 2, b = blockIdx.x;
   const uint64_t g = b < half ? 2 * b : 2 * (b - half) + 1;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const uint32_t D = a.head_dim, nq = D / 4, ng = D / 16;
+  const uint32_t D = DT ? DT : a.head_dim, nq = D / 4, ng = D / 16;
   const bool rans = a.codec == CF_KV_CODEC_RANS_HYBRID;
   // Every per-unit field depends only on g, so all of them are requested at once (one memory latency), and each
   // wavefront starts loading its page's K/V right after (a second one) before any barrier.
@@ -220,7 +284,7 @@ __global__ void __launch_bounds__(kEncThreads) encode_kernel(EncodeArgs a) {
   }
   if (rans) {  // head validated above: tables 2 head and 2 head + 1 exist
     for (int i = tid; i < 512; i += kEncThreads)
-      s_tab[i >> 8][i & 255] = a.ctab[(2ull * head + (i >> 8)) * 256 + (i & 255)];
+      s_tab[i >> 8][i & 255] = reinterpret_cast<const uint2 *>(a.ctab)[(2ull * head + (i >> 8)) * 256 + (i & 255)];
   }
 
   // ---- phase 1: wavefront (X, G) quantises page G of K and V of group X of the unit
@@ -240,18 +304,20 @@ __global__ void __launch_bounds__(kEncThreads) encode_kernel(EncodeArgs a) {
       }
     }
     m = wave_max(m);
-    const float ks = m == 0.0f ? 1.0f : m / 127.0f;
+    const uint32_t absent = rans ? 0u : 0x80808080u;  // the symbol 0 of absent tokens
+    auto inexact = [](float sc) { return !(sc >= 7.8886e-31f && sc <= 1.2677e30f); };  // outside [2^-100, 2^100]
+    const float ks = m == 0.0f ? 1.0f : m / 127.0f, rks = 1.0f / ks;
+    const bool kx_exact = inexact(ks);
 #pragma unroll
     for (int r = 0; r < 8; ++r) {
       const uint32_t i = r * 64 + lane;
       if (i < 4 * D) {
         const uint32_t t = i / nq, q = i % nq;
-        uint32_t w = 0x80808080u;
+        uint32_t w = absent;
         if (t < tc) {
-          const uint32_t b0 = quant8(kx[r].x, ks), b1 = quant8(kx[r].y, ks), b2 = quant8(kx[r].z, ks),
-                         b3 = quant8(kx[r].w, ks);
-          minus |= b0 == 0 || b1 == 0 || b2 == 0 || b3 == 0;
-          w = b0 | b1 << 8 | b2 << 16 | b3 << 24;
+          const float x4[4] = {kx[r].x, kx[r].y, kx[r].z, kx[r].w};
+          w = quant_word(x4, ks, rks, kx_exact, rans);
+          minus |= has_minus128(w, rans);
         }
         kS[X][(G * 16 + t) * kKStride + q] = w;
       }
@@ -265,20 +331,21 @@ __global__ void __launch_bounds__(kEncThreads) encode_kernel(EncodeArgs a) {
         if (d < D && static_cast<uint32_t>(t) < tc) m = __builtin_fmaxf(m, __builtin_fabsf(vx[r][t]));
     }
     m = wave_max(m);
-    const float vs = m == 0.0f ? 1.0f : m / 127.0f;
+    const float vs = m == 0.0f ? 1.0f : m / 127.0f, rvs = 1.0f / vs;
+    const bool vx_exact = inexact(vs);
 #pragma unroll
     for (int r = 0; r < 2; ++r) {
       const uint32_t d = r * 64 + lane;
       if (d < D) {
 #pragma unroll
         for (int tq = 0; tq < 4; ++tq) {
-          uint32_t w = 0;
+          uint32_t w = absent;
+          if (static_cast<uint32_t>(4 * tq) < tc) {
+            float x4[4];
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const uint32_t t = 4 * tq + i;
-            const uint32_t b = t < tc ? quant8(vx[r][t], vs) : 128u;
-            minus |= b == 0;
-            w |= b << (8 * i);
+            for (int i = 0; i < 4; ++i) x4[i] = static_cast<uint32_t>(4 * tq + i) < tc ? vx[r][4 * tq + i] : 0.0f;
+            w = quant_word(x4, vs, rvs, vx_exact, rans);
+            minus |= has_minus128(w, rans);
           }
           vT[X][(G * kMaxDim + d) * kVStride + tq] = w;
         }
@@ -307,12 +374,17 @@ __global__ void __launch_bounds__(kEncThreads) encode_kernel(EncodeArgs a) {
     for (int li = static_cast<int>(nlist) - 1; li >= 0; --li) {
       const uint32_t X = list[li];
       uint32_t base = 0;
-      for (int p = static_cast<int>(D / 8) - 1; p >= 0; --p) {
+      // the table entry of a step does not depend on the state: read one step ahead
+      auto entry = [&](int p) {
         const uint32_t w0 = s == 0 ? k_word(kS[X], G, t, 2 * p) : v_word(vT[X], G, t, 2 * p, ng);
         const uint32_t w1 = s == 0 ? k_word(kS[X], G, t, 2 * p + 1) : v_word(vT[X], G, t, 2 * p + 1, ng);
-        const uint32_t e = s_tab[s][bigs_of(w0) | bigs_of(w1) << 4];
-        const uint32_t f = e & 0xFFFFu, cum = e >> 16;
-        const bool emit = static_cast<uint64_t>(x) >= (static_cast<uint64_t>(f) << 21);  // (2^16 >> 11) << 16
+        return s_tab[s][bigs_of(w0) | bigs_of(w1) << 4];
+      };
+      uint2 e = entry(static_cast<int>(D / 8) - 1);
+      for (int p = static_cast<int>(D / 8) - 1; p >= 0; --p) {
+        const uint2 next = entry(max(p - 1, 0));
+        const uint32_t f = e.x & 0xFFFFu, cum = e.x >> 16;
+        const bool emit = (x >> 21) >= f;  // x >= f << 21 ((2^16 >> 11) << 16)
         const uint64_t mask = __ballot(emit);
         if (emit) {
           const uint32_t above = __popcll(mask & ~((2ull << lane) - 1ull));  // emitters at higher lanes go first
@@ -320,7 +392,10 @@ __global__ void __launch_bounds__(kEncThreads) encode_kernel(EncodeArgs a) {
           x >>= 16;
         }
         base += __popcll(mask);
-        x = ((x / f) << CF_KV_RANS_PROB_BITS) + (x % f) + cum;
+        uint32_t q, r;
+        rans_div(x, f, e.y, q, r);
+        x = (q << CF_KV_RANS_PROB_BITS) + r + cum;
+        e = next;
       }
       if (lane == 0) s_count[s][X] = base;
     }
@@ -336,18 +411,9 @@ __global__ void __launch_bounds__(kEncThreads) encode_kernel(EncodeArgs a) {
       for (int k = 0; k < 8; ++k) {
         const int q = 8 * sg + k;
         const uint32_t w = s == 0 ? k_word(kS[X], G, t, q) : v_word(vT[X], G, t, q, ng);
-        uint32_t nib = 0, cr = 0, sn = 0;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const uint32_t b = (w >> (8 * i)) & 255u;
-          const uint32_t mag = b >= 128u ? b - 128u : 128u - b;
-          nib |= (mag & 15u) << (8 * i);
-          cr |= ((mag >> 4) & 3u) << (8 * i + 4);
-          sn |= (b < 128u ? 1u : 0u) << (8 * i + 7);
-        }
-        wd[kNWord[k]] |= rotl(nib, kFrame[k]);
-        wd[k < 4 ? 2 : 5] |= rotl(cr, kFrame[k]);
-        wd[6] |= rotl(sn, kFrame[k]);
+        wd[kNWord[k]] |= rotl(w & 0x0F0F0F0Fu, kFrame[k]);
+        wd[k < 4 ? 2 : 5] |= rotl(w & 0x30303030u, kFrame[k]);
+        wd[6] |= rotl(w & 0x80808080u, kFrame[k]);
       }
 #pragma unroll
       for (int w = 0; w < 7; ++w) out[(7 * sg + w) * 64 + lane] = wd[w];
@@ -366,7 +432,8 @@ __global__ void __launch_bounds__(kEncThreads) encode_kernel(EncodeArgs a) {
       uint32_t *out = reinterpret_cast<uint32_t *>(blob + kHeader);
       for (uint32_t i = tid; i < 2 * nq * 64; i += kEncThreads) {
         const uint32_t s = i / (nq * 64), r = i % (nq * 64), q = r / 64, L = r % 64;
-        out[i] = s == 0 ? k_word(kS[X], L >> 4, L & 15, q) : v_word(vT[X], L >> 4, L & 15, q, ng);
+        const uint32_t w = s == 0 ? k_word(kS[X], L >> 4, L & 15, q) : v_word(vT[X], L >> 4, L & 15, q, ng);
+        out[i] = rans ? offset_binary(w) : w;
       }
       size = kHeader + 2ull * nq * 64 * 4;
     } else {
@@ -449,7 +516,7 @@ Layout layout_of(uint32_t codec, uint32_t head_dim, uint64_t ngroups, uint32_t t
     at = (at + bytes + 255) & ~uint64_t(255);
     return o;
   };
-  L.ctab = take(static_cast<uint64_t>(table_count) * 256 * 4);
+  L.ctab = take(static_cast<uint64_t>(table_count) * 256 * 8);
   L.tvalid = take(static_cast<uint64_t>(table_count) * 4);
   L.units = take((ngroups + 1) * 4);
   L.offs = take((ngroups + 1) * 4);
@@ -502,7 +569,10 @@ extern "C" cf_status cf_kv_encode_groups_async(uint32_t codec, const float *keys
   if (cfd::launch_status() != CF_OK) return CF_ERR_CUDA;
   EncodeArgs a{keys, values, first_page, page_counts, token_counts, heads, continues, ctab, tvalid, ngroups,
                table_count, codec, head_dim, ws + L.stage, L.cap, units, status};
-  encode_kernel<<<static_cast<unsigned>(ngroups), kEncThreads, 0, st>>>(a);
+  const unsigned wgs = static_cast<unsigned>(ngroups);
+  if (head_dim == 128) encode_kernel<128><<<wgs, kEncThreads, 0, st>>>(a);
+  else if (head_dim == 64) encode_kernel<64><<<wgs, kEncThreads, 0, st>>>(a);
+  else encode_kernel<0><<<wgs, kEncThreads, 0, st>>>(a);
   if (cfd::launch_status() != CF_OK) return CF_ERR_CUDA;
   size_t scan_bytes = L.scan_bytes;
   if (hipcub::DeviceScan::ExclusiveSum(ws + L.scan, scan_bytes, units, offs, static_cast<int>(ngroups + 1), st) !=
