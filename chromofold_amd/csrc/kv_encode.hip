@@ -83,17 +83,26 @@ __global__ void __launch_bounds__(256) table_prep_kernel(const uint8_t *__restri
     units[ngroups] = 0;  // the scan's extra element: its exclusive sum is the pool total
   }
   if (blockIdx.x >= table_count) return;
-  const uint32_t *blob = reinterpret_cast<const uint32_t *>(tables + static_cast<uint64_t>(blockIdx.x) * kTableBytes);
+  // all of a thread's slots in one memory latency (thread t: slots 2 t + 512 k and + 1)
+  typedef uint32_t slot2_t __attribute__((ext_vector_type(4), aligned(4)));  // two slots; blobs may be 4-byte aligned
+  const slot2_t *blob = reinterpret_cast<const slot2_t *>(tables + static_cast<uint64_t>(blockIdx.x) * kTableBytes);
+  slot2_t e[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) e[k] = blob[tid + 256 * k];
   s_last[tid] = -1;
   if (tid == 0) s_total = s_bad = 0;
   __syncthreads();
-  for (int s = tid; s < 2048; s += 256) {
-    const uint32_t lo = blob[2 * s];
-    if (((lo >> 11) & 2047u) == 0) atomicMax(&s_last[(lo >> 22) & 255u], s);
-  }
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const uint32_t lo = h ? e[k].z : e[k].x, slot = 2 * (tid + 256 * k) + h;
+      // the last slot with offset 0 wins: its slot number above, its frequency below
+      if (((lo >> 11) & 2047u) == 0) atomicMax(&s_last[(lo >> 22) & 255u], static_cast<int>(slot << 11 | (lo & 2047u)));
+    }
   __syncthreads();
-  const int s = s_last[tid];
-  const uint32_t f = s < 0 ? 0u : (blob[2 * s] & 2047u);
+  const int won = s_last[tid], s = won < 0 ? -1 : won >> 11;
+  const uint32_t f = won < 0 ? 0u : static_cast<uint32_t>(won) & 2047u;
   if (f == 0) atomicOr(&s_bad, 1u);
   atomicAdd(&s_total, f);
   // {freq | cum << 16, floor(2^32 / freq)}: the coder's division (see rans_div)
