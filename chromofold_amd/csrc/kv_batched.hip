@@ -463,7 +463,9 @@ __device__ __forceinline__ uint32_t span_owner(uint32_t x, uint32_t pairs, uint3
   return div_wide(static_cast<uint64_t>(x + 1) * nwg - 1, pairs);
 }
 
-template <int D, int CODEC, int W>
+// AFTER: the workgroup is the only one of a cascade row and finishes it with the prefix states of slots 0 .. slot0 - 1
+// (a kernel of its own: in the ordinary one that code costs a single sequence's decode 0.3 of 17.2 us).
+template <int D, int CODEC, int W, bool AFTER = false>
 __global__ CF_KV_OCC __launch_bounds__(64 * W) void kv_batched_kernel(cf_kv_batched_desc d, uint32_t splits,
                                                                        float *__restrict__ partial, SplitSlots ss) {
   constexpr int NQ = D / 4;
@@ -741,10 +743,53 @@ __global__ CF_KV_OCC __launch_bounds__(64 * W) void kv_batched_kernel(cf_kv_batc
         o += rw[h * (D + 2) + dd] * sc;
       }
     if (nan) m = __builtin_nanf("");
-    if (ss.slots == 1) {
+    if (!AFTER && ss.slots == 1) {
       if (static_cast<uint32_t>(h) < gqa)
         d.output[(static_cast<size_t>(seq) * d.query_head_count + head * gqa + h) * D + dd] =
             nan ? m : l > 0.0f ? o / l : 0.0f;
+    } else if (AFTER) {
+      // the merge kernel's order and rules, beside the other workgroups' decode
+      const float *pp = partial + (static_cast<size_t>(seq) * d.kv_head_count + head) * ss.slots * (kGqa * (D + 2)) + h * (D + 2);
+      constexpr uint32_t kB = 4;
+      float mm = m;
+      for (uint32_t s0 = 0; s0 < ss.slot0; s0 += kB) {
+        float ms[kB];
+#pragma unroll
+        for (uint32_t u = 0; u < kB; ++u) ms[u] = pp[min(s0 + u, ss.slot0 - 1) * (kGqa * (D + 2)) + D];
+#pragma unroll
+        for (uint32_t u = 0; u < kB; ++u) {
+          nan |= ms[u] != ms[u];
+          mm = fmaxf(mm, ms[u]);
+        }
+      }
+      float lt = 0.0f, ot = 0.0f;
+      if (mm != -INFINITY) {
+        for (uint32_t s0 = 0; s0 < ss.slot0; s0 += kB) {
+          float mq[kB], lq[kB], oq[kB];
+#pragma unroll
+          for (uint32_t u = 0; u < kB; ++u) {
+            const float *q = pp + min(s0 + u, ss.slot0 - 1) * (kGqa * (D + 2));
+            mq[u] = q[D];
+            lq[u] = q[D + 1];
+            oq[u] = q[dd];
+          }
+#pragma unroll
+          for (uint32_t u = 0; u < kB; ++u) {
+            if (s0 + u >= ss.slot0 || mq[u] == -INFINITY) continue;
+            const float sc = __expf(mq[u] - mm);
+            lt += lq[u] * sc;
+            ot += oq[u] * sc;
+          }
+        }
+        if (m != -INFINITY) {
+          const float sc = __expf(m - mm);
+          lt += l * sc;
+          ot += o * sc;
+        }
+      }
+      if (static_cast<uint32_t>(h) < gqa)
+        d.output[(static_cast<size_t>(seq) * d.query_head_count + head * gqa + h) * D + dd] =
+            nan ? __builtin_nanf("") : lt == 0.0f ? 0.0f : ot / lt;
     } else {
       float *pp = partial + ((static_cast<size_t>(seq) * d.kv_head_count + head) * ss.slots + ss.slot0 + split) *
                                 (kGqa * (D + 2));
@@ -1225,12 +1270,18 @@ __global__ __launch_bounds__(kGqa * D) void kv_span_merge_kernel(cf_kv_batched_d
 //   scores   S^T = K Q^T per 16-token page: A = K[token][8 dims] (two raw u32 quads, converted exactly to f16 as
 //            (1024 + sym) - 1152), B = Q^T (hi and lo f16 parts held in registers), scaled by the page's K scale;
 //            the lane's accumulator registers hold S^T[tokens 4kg + r][row lane & 15];
-//   softmax  online per row (its values live in the 4 lanes sharing lane & 15);
+//   softmax  online per row (its values live in the 4 lanes sharing lane & 15), O rescaled only when a row's maximum
+//            passes the reference by ln 2;
 //   P V      those same registers ARE the A operand of the P V product when the k index of a 32-token step is
 //            ordered {4kg + r of page 2s, 4kg + r of page 2s + 1}: no transpose. B = V[those tokens][dim] is two raw
 //            u32 V quads of the INT8 layout as they are; P is pre-multiplied by each page's V scale and split into
 //            f16 hi + lo parts, one MFMA each (one f16 per weight loses near-cancelling outputs).
 // Operands: each group is converted once per workgroup into double-buffered LDS (see the kernel body).
+// Bound: the vector work of a group (softmax, f16 parts, conversion: half of the wave's time) beside its 64 matrix
+// instructions (a third), on two waves per SIMD. 256 sequences x 8 heads x 8192 tokens: 117 us with AGPR copies, a
+// rescale per group, scalar header loads and a query row in 32 loads; 93-97 us without. Two row tiles per wave halve the
+// operand reads and need twice the prefix states (97-100 us and a slower merge; on one wave per SIMD 112 us), scores
+// of the next group beside the weights of this one change nothing (98 us), eight waves per workgroup neither (100 us).
 // A non-INT8 group in the prefix makes the prefix partials NaN, so every output is NaN (the prefix must be raw).
 
 __device__ __forceinline__ half8_t sym8_to_f16(uint32_t w0, uint32_t w1) {
@@ -1249,47 +1300,70 @@ __device__ __forceinline__ half8_t sym8_to_f16(uint32_t w0, uint32_t w1) {
   return r;
 }
 
+typedef float float4u_t __attribute__((ext_vector_type(4), aligned(4)));
 constexpr int kPfxThreads = 256;  // 4 waves x 16 rows = 16 sequences per workgroup
 
-__global__ __launch_bounds__(kPfxThreads) void kv_prefix_kernel(cf_kv_batched_desc d, uint32_t shared,
-                                                                 uint32_t psplits, float *__restrict__ partial,
-                                                                 SplitSlots ss) {
+__global__ __launch_bounds__(kPfxThreads) __attribute__((amdgpu_waves_per_eu(2))) void kv_prefix_kernel(
+    cf_kv_batched_desc d, uint32_t shared, uint32_t psplits, float *__restrict__ partial, SplitSlots ss) {
   constexpr int D = 128, NQ = D / 4;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int j = lane & 15, kg = lane >> 4;
-  const uint32_t head = blockIdx.y, psplit = blockIdx.z;
+  // workgroups that read the same groups (the row tiles of a (head, split) unit) are 8 apart, on one XCD's L2; the
+  // units beyond a multiple of 8 follow tile by tile
+  const uint32_t tiles = (d.seq_count + 15) / 16, units8 = d.kv_head_count * psplits / 8 * 8;
+  const bool swz = blockIdx.x < units8 * tiles;
+  const uint32_t rest = blockIdx.x - units8 * tiles;
+  const uint32_t tile = swz ? blockIdx.x / 8 % tiles : rest % tiles;
+  const uint32_t unit = swz ? blockIdx.x / 8 / tiles * 8 + blockIdx.x % 8 : units8 + rest / tiles;
+  const uint32_t head = unit % d.kv_head_count, psplit = unit / d.kv_head_count;
   const uint32_t gqa = d.query_head_count / d.kv_head_count;
-  const uint32_t rseq = blockIdx.x * 16 + wave * 4 + j / 4, rh = j % 4;  // the lane's row j
+  const uint32_t rseq = tile * 16 + wave * 4 + j / 4, rh = j % 4;  // the lane's row j
   const bool row_ok = rseq < d.seq_count && rh < gqa;
-
-  // Q^T operand: B[dims 32ks + 8kg .. +7][row j], split into f16 hi + lo parts (fp32-grade scores)
-  half8_t qh[4], ql[4];
-#pragma unroll
-  for (int ks = 0; ks < 4; ++ks)
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float q = row_ok ? d.queries[(static_cast<size_t>(rseq) * d.query_head_count + head * gqa + rh) * D +
-                                         32 * ks + 8 * kg + e]
-                             : 0.0f;
-      _Float16 h, l;
-      cfd::split_mul_f16(q, d.softmax_scale, h, l);
-      qh[ks][e] = h;
-      ql[ks][e] = l;
-    }
-  const uint32_t vis = row_ok ? min(d.seq_tokens[rseq], d.query_pos[rseq] + 1) : 0u;
-  // wave-wide: the fewest visible tokens over the valid rows (invalid rows are never written)
-  uint32_t vmin = row_ok ? vis : 0xFFFFFFFFu;
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) vmin = min(vmin, static_cast<uint32_t>(__shfl_xor(static_cast<int>(vmin), o)));
 
   const uint32_t per = (shared + psplits - 1) / psplits;
   const uint32_t ga = min(shared, psplit * per), gb = min(shared, ga + per);
   const uint32_t *grow = d.group_offsets + static_cast<size_t>(head) * d.max_groups;  // sequence 0's table
+  // Word lane & 15 of a group's 64-byte header, and a group's offset, as vector loads (a scalar load would be waited
+  // for with the next LDS access): headers are loaded two groups ahead of their use, offsets three.
+  uint32_t zero = 0;
+  asm volatile("" : "+v"(zero));
+  auto offset_at = [&](uint32_t g) { return grow[min(g, gb - 1) + zero]; };
+  auto header_at = [&](uint32_t off) { return reinterpret_cast<const uint32_t *>(d.pool + static_cast<size_t>(off) * 16)[j]; };
+  // requested before the query rows, so that the chain offset - header - words runs beside them
+  uint32_t off0 = 0, off1 = 0, off2 = 0, hdr = 0, hdr1 = 0;  // offsets of g .. g + 2; header words of g, g + 1
+  if (ga < gb) {
+    off0 = offset_at(ga);
+    off1 = offset_at(ga + 1);
+    off2 = offset_at(ga + 2);
+    hdr = header_at(off0);
+    hdr1 = header_at(off1);
+  }
 
-  float m = -INFINITY, l = 0.0f;  // row j's running max / sum (same in the 4 lanes of the row)
-  bool coded = false;              // a prefix group that is not INT8 was met
-  int e_run = -(1 << 20);          // acc is kept in units of 2^e_run (e_run: V-scale exponent of the current group)
-  float4_t acc[D / 16];            // O[rows 4kg + r][dims 16 dt + j]
+  // Q^T operand: B[dims 32ks + 8kg .. +7][row j], split into f16 hi + lo parts (fp32-grade scores)
+  half8_t qh[4], ql[4];
+  const float *q = d.queries +
+                   (static_cast<size_t>(row_ok ? rseq : 0) * d.query_head_count + head * gqa + (row_ok ? rh : 0)) * D;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const float4u_t v = *reinterpret_cast<const float4u_t *>(q + 32 * (i / 2) + 8 * kg + 4 * (i % 2));
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      _Float16 h, l;
+      cfd::split_mul_f16(row_ok ? v[e] : 0.0f, d.softmax_scale, h, l);
+      qh[i / 2][4 * (i % 2) + e] = h;
+      ql[i / 2][4 * (i % 2) + e] = l;
+    }
+  }
+  const uint32_t vis = row_ok ? min(d.seq_tokens[rseq], d.query_pos[rseq] + 1) : 0u;
+  uint32_t vmin = row_ok ? vis : 0xFFFFFFFFu;  // the fewest visible tokens over the wave's rows
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) vmin = min(vmin, static_cast<uint32_t>(__shfl_xor(static_cast<int>(vmin), o)));
+
+  float m = -INFINITY;      // row j's softmax reference (same in its 4 lanes), at most ln 2 below the running maximum
+  float l = 0.0f;           // the lane's share of row j's sum (its 4 lanes are added at the end)
+  int e_run = -(1 << 20);   // acc is kept in units of 2^e_run (from the V-scale exponents of the groups)
+  bool coded = false;       // a prefix group that is not INT8 was met
+  float4_t acc[D / 16];     // O[rows 4kg + r][dims 16 dt + j]
 #pragma unroll
   for (int dt = 0; dt < D / 16; ++dt) acc[dt] = float4_t{0, 0, 0, 0};
 
@@ -1298,22 +1372,21 @@ __global__ __launch_bounds__(kPfxThreads) void kv_prefix_kernel(cf_kv_batched_de
   // buffers; the next group's raw words are loaded while the current group is computed from the other buffer.
   __shared__ half8_t s_op[2][2][16][64];  // [buffer][K, V][slot][lane], 64 KiB
   uint32_t w[16];
-  auto codec_at = [&](uint32_t g) { return *reinterpret_cast<const uint32_t *>(d.pool + static_cast<size_t>(grow[g]) * 16); };
-  // raw words of group g; a group that is not INT8 (smaller blob: reading an INT8-sized span could run past the
-  // pool) is not read, its outputs become NaN anyway
-  auto fetch = [&](uint32_t g, bool raw_group) {
-    const uint32_t *raw = reinterpret_cast<const uint32_t *>(d.pool + static_cast<size_t>(grow[g]) * 16 + kHdr);
-    if (!raw_group) {
+  // raw words of a group; one that is not INT8 (smaller blob: reading an INT8-sized span could run past the pool) is
+  // not read, its outputs become NaN anyway
+  auto fetch = [&](uint32_t off, uint32_t hdr) {
+    if (__builtin_amdgcn_readfirstlane(hdr) != CF_KV_CODEC_INT8) {
 #pragma unroll
       for (int i = 0; i < 16; ++i) w[i] = 0;
       return;
     }
+    const uint32_t *raw = reinterpret_cast<const uint32_t *>(
+        d.pool + static_cast<size_t>(static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(off))) * 16 + kHdr);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int ks_slot = 4 * wave + i, G = ks_slot / 4, ks = ks_slot % 4;
-      w[2 * i] = raw[(8 * ks + 2 * kg) * 64 + 16 * G + j];
-      w[2 * i + 1] = raw[(8 * ks + 2 * kg + 1) * 64 + 16 * G + j];
-      const int v_slot = 4 * wave + i, s2 = v_slot / 8, dt = v_slot % 8;
+      w[2 * i] = raw[(8 * i + 2 * kg) * 64 + 16 * wave + j];
+      w[2 * i + 1] = raw[(8 * i + 2 * kg + 1) * 64 + 16 * wave + j];
+      const int s2 = wave / 2, dt = (4 * wave + i) % 8;
       w[8 + 2 * i] = raw[NQ * 64 + (kg * (D / 16) + dt) * 64 + 16 * (2 * s2) + j];
       w[9 + 2 * i] = raw[NQ * 64 + (kg * (D / 16) + dt) * 64 + 16 * (2 * s2 + 1) + j];
     }
@@ -1325,119 +1398,123 @@ __global__ __launch_bounds__(kPfxThreads) void kv_prefix_kernel(cf_kv_batched_de
       s_op[buf][1][4 * wave + i][lane] = sym8_to_f16(w[8 + 2 * i], w[9 + 2 * i]);
     }
   };
-  // the codec of group g + 1 is loaded one group ahead of its fetch, so the fetch does not wait for it
-  uint32_t codec_next = ga + 1 < gb ? codec_at(ga + 1) : 0u;
   if (ga < gb) {
-    fetch(ga, codec_at(ga) == CF_KV_CODEC_INT8);
+    fetch(off0, hdr);
     store(0);
   }
   __syncthreads();
   for (uint32_t g = ga; g < gb; ++g) {
     const int buf = (g - ga) & 1;
-    const uint32_t codec1 = codec_next;
-    if (g + 2 < gb) codec_next = codec_at(g + 2);
-    if (g + 1 < gb) fetch(g + 1, codec1 == CF_KV_CODEC_INT8);
-    const uint8_t *blob = d.pool + static_cast<size_t>(grow[g]) * 16;
-    const uint32_t codec = *reinterpret_cast<const uint32_t *>(blob);
-    const uint32_t tc01 = *reinterpret_cast<const uint32_t *>(blob + 12), tc23 = *reinterpret_cast<const uint32_t *>(blob + 16);
-    const float *kscale = reinterpret_cast<const float *>(blob + 32), *vscale = reinterpret_cast<const float *>(blob + 48);
-    const bool full = tc01 == 0x00100010u && tc23 == 0x00100010u;
-    coded |= codec != CF_KV_CODEC_INT8;
-    const bool fast = full && vmin >= 64u * (g + 1);  // every row sees every token of the group
+    const uint32_t hdr2 = header_at(off2), off3 = offset_at(g + 3);
+    if (g + 1 < gb) fetch(off1, hdr1);
+    auto word = [&](int i) { return static_cast<uint32_t>(__builtin_amdgcn_readlane(hdr, i)); };
+    const uint32_t tc01 = word(3), tc23 = word(4);
+    coded |= word(0) != CF_KV_CODEC_INT8;
     float4_t st[4];
 #pragma unroll
     for (int G = 0; G < 4; ++G) {
-      float4_t acc_s = {0, 0, 0, 0};
+      float4_t a = {0, 0, 0, 0};
 #pragma unroll
       for (int ks = 0; ks < 4; ++ks) {
         const half8_t kf = s_op[buf][0][4 * G + ks][lane];
-        acc_s = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, qh[ks], acc_s, 0, 0, 0);
-        acc_s = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, ql[ks], acc_s, 0, 0, 0);
+        a = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, qh[ks], a, 0, 0, 0);
+        a = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, ql[ks], a, 0, 0, 0);
       }
-      const float ksc = kscale[G];
+      const float ksc = __uint_as_float(word(8 + G));
 #pragma unroll
-      for (int r = 0; r < 4; ++r) st[G][r] = acc_s[r] * ksc;
-      if (!fast) {
+      for (int r = 0; r < 4; ++r) st[G][r] = a[r] * ksc;
+    }
+    // unless every row sees every token of the group
+    if (tc01 != 0x00100010u || tc23 != 0x00100010u || vmin < 64u * (g + 1)) {
+#pragma unroll
+      for (int G = 0; G < 4; ++G) {
         const uint32_t tcg = (G < 2 ? tc01 : tc23) >> (16 * (G & 1)) & 0xFFFFu;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const uint32_t t = 4 * kg + r;
-          if (t >= tcg || 64u * g + 16u * G + t >= vis) st[G][r] = -INFINITY;
+          const uint32_t tok = 4 * kg + r;
+          if (tok >= tcg || 64u * g + 16u * G + tok >= vis) st[G][r] = -INFINITY;
         }
       }
     }
-    // online softmax of row j over the group's 64 tokens
+    // P V units: O is kept in units of 2^e_run with e_run >= (exponent of the group's largest present-page V scale)
+    // - 14, so the f16 operand p * v_scale * 2^-e_run stays below 2^15 whatever the V magnitude and weights down to
+    // 2^-25 of the running maximum stay normal
+    float vscale[4], vmax = 0.0f;
+#pragma unroll
+    for (int G = 0; G < 4; ++G) {
+      vscale[G] = __uint_as_float(word(12 + G));
+      if (((G < 2 ? tc01 : tc23) >> (16 * (G & 1)) & 0xFFFFu) != 0u) vmax = fmaxf(vmax, vscale[G]);
+    }
+    const int ev = __builtin_amdgcn_readfirstlane(__builtin_amdgcn_frexp_expf(vmax)) - 14;
+    // Online softmax of row j over the group's 64 tokens. The reference m and the units move only when a row's
+    // maximum passes m by more than ln 2 (p stays <= 2) or the V exponent rises, or falls by more than 2: most groups
+    // then skip the rescale of O.
     float mx = -INFINITY;
 #pragma unroll
     for (int G = 0; G < 4; ++G)
 #pragma unroll
       for (int r = 0; r < 4; ++r) mx = fmaxf(mx, st[G][r]);
     mx = cfd::rows4_max(mx);
-    const float mn = fmaxf(m, mx);
-    const float alpha = m == -INFINITY ? 0.0f : __expf(m - mn);
-    m = mn;
-    float psum = 0.0f;
-#pragma unroll
-    for (int G = 0; G < 4; ++G)
+    if (__ballot(mx > m + 0.6931f) || ev > e_run || ev < e_run - 2) {
+      const float mn = fmaxf(m, mx);
+      const float alpha = m == -INFINITY ? 0.0f : __expf(m - mn);
+      m = mn;
+      l *= alpha;
+      // moving to the group's units is an exact power of two (a drop of more than 2^60 is clamped)
+      const int en = max(ev, e_run - 60), de = e_run - en;
+      e_run = en;
+      // O's rows are 4kg + r, whose alpha lives in lane 4kg + r
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const float p = st[G][r] == -INFINITY ? 0.0f : __expf(st[G][r] - mn);
-        st[G][r] = p;
-        psum += p;
+        const float ar = ldexpf(__shfl(alpha, 4 * kg + r), de);
+#pragma unroll
+        for (int dt = 0; dt < D / 16; ++dt) acc[dt][r] *= ar;
       }
-    psum = cfd::rows4_sum(psum);
-    l = l * alpha + psum;
-    // P V units: O is kept in units of 2^e with e = (exponent of the group's largest present-page V scale) - 15,
-    // so the f16 operand p * v_scale * 2^-e stays below 2^15 whatever the V magnitude and weights down to 2^-29
-    // of the running maximum stay normal; moving to the group's units is an exact power-of-two factor folded into
-    // the softmax rescale (a drop of more than 2^60 is clamped)
-    float vmax = 0.0f;
-#pragma unroll
-    for (int G = 0; G < 4; ++G)
-      if (((G < 2 ? tc01 : tc23) >> (16 * (G & 1)) & 0xFFFFu) != 0u) vmax = fmaxf(vmax, vscale[G]);
-    const int ev = max(__builtin_amdgcn_frexp_expf(vmax) - 15, e_run - 60);
-    const int de = e_run - ev;
-    e_run = ev;
-    // rescale O: its rows are 4kg + r, whose alpha lives in lane 4kg + r
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const float ar = ldexpf(__shfl(alpha, 4 * kg + r), de);
-#pragma unroll
-      for (int dt = 0; dt < D / 16; ++dt) acc[dt][r] *= ar;
     }
     // P V over page pairs (2s, 2s + 1); the weights p * v_scale as f16 hi + lo parts
 #pragma unroll
     for (int s2 = 0; s2 < 2; ++s2) {
-      half8_t pa, pl;
-      const float v0 = ldexpf(vscale[2 * s2], -ev), v1 = ldexpf(vscale[2 * s2 + 1], -ev);
+      half8_t ph, pl;
+      const float mref = m == -INFINITY ? 0.0f : m;  // no token visible yet: every p is exp(-inf) = 0
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        _Float16 h, lo;
-        cfd::split_mul_f16(st[2 * s2][r], v0, h, lo);
-        pa[r] = h;
-        pl[r] = lo;
-        cfd::split_mul_f16(st[2 * s2 + 1][r], v1, h, lo);
-        pa[4 + r] = h;
-        pl[4 + r] = lo;
+      for (int u = 0; u < 2; ++u) {
+        const float v = ldexpf(vscale[2 * s2 + u], -e_run);
+#pragma unroll
+        for (int r = 0; r < 4; r += 2) {
+          const float p0 = __expf(st[2 * s2 + u][r] - mref), p1 = __expf(st[2 * s2 + u][r + 1] - mref);
+          l += p0;
+          l += p1;
+          _Float16 a0, b0, a1, b1;
+          cfd::split2_mul_f16(p0, p1, v, a0, b0, a1, b1);
+          ph[4 * u + r] = a0;
+          pl[4 * u + r] = b0;
+          ph[4 * u + r + 1] = a1;
+          pl[4 * u + r + 1] = b1;
+        }
       }
 #pragma unroll
       for (int dt = 0; dt < D / 16; ++dt) {
         const half8_t vb = s_op[buf][1][8 * s2 + dt][lane];
-        acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa, vb, acc[dt], 0, 0, 0);
+        acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ph, vb, acc[dt], 0, 0, 0);
         acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pl, vb, acc[dt], 0, 0, 0);
       }
     }
     if (g + 1 < gb) store(buf ^ 1);  // the other buffer: every wave finished with it before the last barrier
     __syncthreads();
+    hdr = hdr1;
+    hdr1 = hdr2;
+    off1 = off2;
+    off2 = off3;
   }
 
   // partial state of rows 4kg + r (m and l from lane 4kg + r) into slot psplit
+  l = cfd::rows4_sum(l);
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const int row = 4 * kg + r;
     // a coded prefix group makes the partial NaN, which the merge carries into the output
     const float mr = coded ? __builtin_nanf("") : __shfl(m, row), lr = coded ? __builtin_nanf("") : __shfl(l, row);
-    const uint32_t seq = blockIdx.x * 16 + wave * 4 + row / 4, h = row % 4;
+    const uint32_t seq = tile * 16 + wave * 4 + row / 4, h = row % 4;
     if (seq >= d.seq_count || h >= gqa) continue;
     float *pp = partial + ((static_cast<size_t>(seq) * d.kv_head_count + head) * ss.slots + ss.slot0 + psplit) *
                               (kGqa * (D + 2)) + h * (D + 2);
@@ -2042,13 +2119,13 @@ void launch_span(const cf_kv_batched_desc &d, uint32_t nwg, void *ws, hipStream_
   kv_span_merge_kernel<D><<<dim3(d.kv_head_count, d.seq_count), kGqa * D, 0, s>>>(d, states, sp);
 }
 
-template <int D, int C>
+template <int D, int C, bool AFTER = false>
 void launch_batched(const cf_kv_batched_desc &d, const BatchedPlan &p, dim3 grid, float *ws, SplitSlots ss,
                     hipStream_t s) {
   if (p.waves == 12)
-    kv_batched_kernel<D, C, kWavesWide><<<grid, 64 * kWavesWide, 0, s>>>(d, p.splits, ws, ss);
+    kv_batched_kernel<D, C, kWavesWide, AFTER><<<grid, 64 * kWavesWide, 0, s>>>(d, p.splits, ws, ss);
   else
-    kv_batched_kernel<D, C, kWavesNarrow><<<grid, 64 * kWavesNarrow, 0, s>>>(d, p.splits, ws, ss);
+    kv_batched_kernel<D, C, kWavesNarrow, AFTER><<<grid, 64 * kWavesNarrow, 0, s>>>(d, p.splits, ws, ss);
 }
 
 }  // namespace
@@ -2139,14 +2216,18 @@ extern "C" cf_status cf_kv_paged_attention_cascade_async(const cf_kv_batched_des
   if (!d->workspace || d->workspace_bytes < need) return CF_ERR_INVALID_ARGUMENT;
   const hipStream_t s = cfd::as_stream(stream);
   float *ws = static_cast<float *>(d->workspace);
-  kv_prefix_kernel<<<dim3((d->seq_count + 15) / 16, d->kv_head_count, p.psplits), kPfxThreads, 0, s>>>(
+  kv_prefix_kernel<<<(d->seq_count + 15) / 16 * d->kv_head_count * p.psplits, kPfxThreads, 0, s>>>(
       *d, shared_groups, p.psplits, ws, SplitSlots{0, 0, p.slots});
   const SplitSlots rest{shared_groups, p.psplits, p.slots};
   const dim3 grid(p.suffix.splits, d->kv_head_count, d->seq_count);
-  if (d->codec == CF_KV_CODEC_RANS_HYBRID)
-    launch_batched<128, CF_KV_CODEC_RANS_HYBRID>(*d, p.suffix, grid, ws, rest, s);
-  else
-    launch_batched<128, CF_KV_CODEC_INT8>(*d, p.suffix, grid, ws, rest, s);
+  const bool rans = d->codec == CF_KV_CODEC_RANS_HYBRID;
+  if (p.suffix.splits == 1) {
+    if (rans) launch_batched<128, CF_KV_CODEC_RANS_HYBRID, true>(*d, p.suffix, grid, ws, rest, s);
+    else launch_batched<128, CF_KV_CODEC_INT8, true>(*d, p.suffix, grid, ws, rest, s);
+    return cfd::launch_status();
+  }
+  if (rans) launch_batched<128, CF_KV_CODEC_RANS_HYBRID>(*d, p.suffix, grid, ws, rest, s);
+  else launch_batched<128, CF_KV_CODEC_INT8>(*d, p.suffix, grid, ws, rest, s);
   kv_merge_kernel<128><<<dim3(d->kv_head_count, d->seq_count), kGqa * 128, 0, s>>>(*d, p.slots, ws);
   return cfd::launch_status();
 }
