@@ -1,6 +1,7 @@
 // kv_batched.hip — batched compressed paged-KV attention decode on gfx950 (kv_codec_ext.h entry point).
 //
-// One workgroup serves one (sequence, KV head, context split): 12 wavefronts (one workgroup per CU) for long
+// A ragged batch runs as spans: one workgroup per CU takes an equal stretch of a KV head's chain pairs, all sequences
+// laid end to end (kv_span_kernel). Otherwise one workgroup serves one (sequence, KV head, context split): 12 wavefronts (one workgroup per CU) for long
 // contexts, 4 (three workgroups per CU) for short ones. In a 12-wavefront workgroup each wavefront takes a contiguous
 // block of the split's chain pairs sized by its issue priority (arbitration favours the oldest wavefront of a SIMD),
 // so that all finish together. Each wavefront walks "page quads": four consecutive 16-token pages, one per 16-lane
@@ -2266,8 +2267,11 @@ cf_status scratch_address(void **out) {
 extern "C" cf_status cf_kv_paged_attention_batched_noalloc_async(const cf_kv_batched_desc *d, void *stream) {
   const cf_status v = cf_kv_validate_batched_desc(d);
   if (v != CF_OK) return v;
+  // spans only where the split launch would use the shared scratch too: a launch that needs none may overlap others
   BatchedPlan plan = batched_plan(d);
-  if (plan.span_wg && plan_workspace_bytes(d, plan) > CF_KV_BATCHED_NOALLOC_SCRATCH_BYTES) plan = split_plan(d);
+  const BatchedPlan split = split_plan(d);
+  if (plan.span_wg && (split.splits == 1 || plan_workspace_bytes(d, plan) > CF_KV_BATCHED_NOALLOC_SCRATCH_BYTES))
+    plan = split;
   const uint64_t need = plan_workspace_bytes(d, plan);
   if (need > CF_KV_BATCHED_NOALLOC_SCRATCH_BYTES) return CF_ERR_UNSUPPORTED;
   void *ws = nullptr;

@@ -5,15 +5,16 @@
 // encode step of the append path (reference src/runtime/compressed_kv_cache.cu:89-109 seals pages on the host), so
 // K/V that the model produced in HBM never leave the device. Three launches on the caller's stream, nothing
 // allocated:
-//   1. table_prep_kernel: one workgroup per table blob derives the compact (freq, cum) pairs of its 256 joint
+//   1. table_prep_kernel: one workgroup per table blob derives freq, cum and the reciprocal of freq of its 256 joint
 //      symbols (last slot with offset 0 wins, exactly the host loader's rule) and whether the table is usable;
 //      workgroup 0 also clears the status word.
 //   2. encode_kernel: one 8-wavefront workgroup per chain unit (a group alone, or a group and the group that
 //      continues its chain; the workgroup of a continuing group only checks its flag). The unit's fields all
 //      depend only on the group index, so they are requested at once, and every wavefront issues its page's K/V
 //      loads before the first barrier (two memory latencies before any compute, not one per field). Phase 1:
-//      wavefront 4 X + G quantises page G of group X (absmax over the page's present tokens, IEEE division, round
-//      half to even) into LDS symbol tiles laid out for the later reads (K token-major, V dim-major, both padded to
+//      wavefront 4 X + G quantises page G of group X (absmax over the page's present tokens, a
+//      reciprocal with IEEE division near a rounding boundary, round half to even) into LDS tiles of sign-magnitude
+//      symbols laid out for the later reads (K token-major, V dim-major, both padded to
 //      odd word strides). Phase 2: wavefronts 0 and 1 rANS-code the K and V chains across the unit's coded groups in
 //      reverse (64 interleaved states each); the renormalisation words of one step are placed with a ballot prefix
 //      count, written from the top of an LDS buffer down so that the reversed stream needs no second pass. At the

@@ -158,6 +158,8 @@ class BatchedKv:
     host_offsets: np.ndarray | None = None
     host_tables: np.ndarray | None = None
     workspace: torch.Tensor | None = None
+    workspace_stream: int | None = None  # the stream whose calls use `workspace`; another stream has its own
+    stream_workspaces: dict = field(default_factory=dict)
     stats: dict = field(default_factory=dict)
 
     @property
@@ -165,9 +167,9 @@ class BatchedKv:
         return int(self.pool.numel())
 
     def desc(self, queries: torch.Tensor, output: torch.Tensor, query_pos: torch.Tensor, softmax_scale: float,
-             splits: int = 0, shared_groups: int = 0) -> cf_kv_batched_desc:
-        """Descriptor (with a workspace of this object's) for attention(); shared_groups > 0 sizes the workspace
-        for the cascade entry point."""
+             splits: int = 0, shared_groups: int = 0, stream=None) -> cf_kv_batched_desc:
+        """Descriptor (with a workspace of this object's for the stream, the current one by default) for attention();
+        shared_groups > 0 sizes the workspace for the cascade entry point."""
         d = cf_kv_batched_desc()
         d.struct_size = C.sizeof(cf_kv_batched_desc)
         d.abi_version = EXT_ABI_VERSION
@@ -193,19 +195,33 @@ class BatchedKv:
         else:
             need = int(A.lib().cf_kv_batched_workspace_bytes(C.byref(d)))
         if need:
-            if self.workspace is None or self.workspace.numel() < need:
-                self.workspace = torch.empty(need, dtype=torch.uint8, device=self.pool.device)
-            d.workspace = self.workspace.data_ptr()
-            d.workspace_bytes = self.workspace.numel()
+            ws = self._stream_workspace(need, (stream if stream is not None else torch.cuda.current_stream()).cuda_stream)
+            d.workspace = ws.data_ptr()
+            d.workspace_bytes = ws.numel()
         return d
+
+    def _stream_workspace(self, need: int, stream: int) -> torch.Tensor:
+        # calls on two streams may overlap, so each stream has a workspace of its own
+        if self.workspace is None or self.workspace_stream is None:
+            self.workspace_stream = stream
+        own = stream == self.workspace_stream
+        ws = self.workspace if own else self.stream_workspaces.get(stream)
+        if ws is None or ws.numel() < need:
+            ws = torch.empty(need, dtype=torch.uint8, device=self.pool.device)
+            if own:
+                self.workspace = ws
+            else:
+                self.stream_workspaces[stream] = ws
+        return ws
 
     def attention(self, queries: torch.Tensor, output: torch.Tensor, query_pos: torch.Tensor,
                   softmax_scale: float, splits: int = 0, stream=None, desc: cf_kv_batched_desc | None = None,
                   shared_groups: int = 0):
         """Batched decode; shared_groups > 0 uses the cascade entry point (the first shared_groups groups of every
         sequence are sequence 0's, stored as INT8 blobs), with a descriptor made by desc(..., shared_groups=)."""
-        d = desc if desc is not None else self.desc(queries, output, query_pos, softmax_scale, splits, shared_groups)
-        s = (stream if stream is not None else torch.cuda.current_stream()).cuda_stream
+        stream = stream if stream is not None else torch.cuda.current_stream()
+        d = desc if desc is not None else self.desc(queries, output, query_pos, softmax_scale, splits, shared_groups, stream)
+        s = stream.cuda_stream
         if shared_groups:
             A.check(A.lib().cf_kv_paged_attention_cascade_async(C.byref(d), shared_groups, s),
                     "cf_kv_paged_attention_cascade_async")

@@ -116,7 +116,8 @@ typedef struct cf_kv_group_header {
  *   query_pos    [seq_count]  position of the decoded query token (causal limit; tokens > query_pos are masked)
  *   queries      [seq_count, query_head_count, head_dim] fp32, output the same shape
  * A shared prefix is expressed by several sequences pointing at the same group blobs (refcounted pages).
- * `workspace` is caller-owned device memory of cf_kv_batched_workspace_bytes() bytes (split-context partials);
+ * `workspace` is caller-owned device memory of cf_kv_batched_workspace_bytes() bytes (span or split-context
+ * partials; with splits = 0 a smaller one, or none, runs a launch that needs less where there is one);
  * the entry point allocates nothing and never synchronises. */
 typedef struct cf_kv_batched_desc {
     uint32_t struct_size;
@@ -140,7 +141,7 @@ typedef struct cf_kv_batched_desc {
     uint64_t workspace_bytes;
 } cf_kv_batched_desc;
 
-/* Bytes of workspace the launch needs for this descriptor (0 when no split is used). Host only. */
+/* Bytes of workspace the launch needs for this descriptor (0 when neither spans nor splits are used). Host only. */
 uint64_t cf_kv_batched_workspace_bytes(const cf_kv_batched_desc *desc);
 
 /* Host-only validation of a batched descriptor (no device dereference). A pool or table pointer that is not
@@ -155,8 +156,8 @@ cf_status cf_kv_paged_attention_batched_async(const cf_kv_batched_desc *desc, vo
  * partials go to a library-owned device array of CF_KV_BATCHED_NOALLOC_SCRATCH_BYTES per GPU instead of
  * desc->workspace (ignored). No counterpart in the reference; it is for callers that cannot allocate device memory
  * (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc). It calls no allocator. A
- * descriptor whose cf_kv_batched_workspace_bytes() exceeds that size returns CF_ERR_UNSUPPORTED (use the workspace
- * entry point, or fewer splits). Every call on one GPU shares that GPU's array: calls that overlap on one GPU
+ * descriptor whose split partials exceed that size returns CF_ERR_UNSUPPORTED (use the workspace entry point, or
+ * fewer splits). Every call on one GPU shares that GPU's array: calls that overlap on one GPU
  * (concurrent streams or threads) race and must be serialised by the caller. */
 #define CF_KV_BATCHED_NOALLOC_SCRATCH_BYTES (8u << 20)
 cf_status cf_kv_paged_attention_batched_noalloc_async(const cf_kv_batched_desc *desc, void *stream);

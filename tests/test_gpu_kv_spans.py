@@ -132,3 +132,31 @@ def test_span_in_a_graph_and_with_a_small_workspace():
     run()
     torch.cuda.synchronize()
     assert float((out - eager).norm() / eager.norm()) <= 1e-5
+
+
+def test_calls_on_two_streams_have_a_workspace_each():
+    """Overlapping calls of one batch on two streams, over shapes that run as spans, give the results of calls in turn."""
+    import torch
+    from chromofold_amd import kv
+    dev = torch.device("cuda:0")
+    rng = np.random.default_rng(6)
+    H, gqa, D, lens = 4, 2, 64, [3000, 200, 900, 64] * 10
+    data = [tuple(rng.standard_normal((H, T, D)).astype(np.float32) for _ in range(2)) for T in lens]
+    kvb = kv.build_batched(kv.CODEC_INT8, lambda s: data[s], len(lens), H, np.array(lens), D, None, dev, encoder="device")
+    pos = torch.tensor(lens, dtype=torch.int32, device=dev) - 1
+    qs = [torch.from_numpy(rng.standard_normal((len(lens), H * gqa, D)).astype(np.float32)).to(dev) for _ in range(2)]
+    want = [torch.empty_like(q) for q in qs]
+    for q, o in zip(qs, want):
+        kvb.attention(q, o, pos, 0.125)
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    ptrs = [kvb.desc(qs[0], want[0], pos, 0.125, stream=s).workspace for s in streams]
+    assert ptrs[0] != ptrs[1] and ptrs[0] == kvb.desc(qs[0], want[0], pos, 0.125, stream=streams[0]).workspace
+    got = [torch.empty_like(q) for q in qs]
+    torch.cuda.synchronize()
+    for _ in range(20):
+        for s, q, o in zip(streams, qs, got):
+            kvb.attention(q, o, pos, 0.125, stream=s)
+    torch.cuda.synchronize()
+    for o, w in zip(got, want):
+        assert torch.equal(o, w)
