@@ -63,3 +63,35 @@ def test_rounding_boundaries(codec, D):
     assert int(r.status.item()) == 0 and int(r.pool_end.item()) == want.size
     assert np.array_equal(r.offsets.cpu().numpy().view(np.uint32), offs)
     assert np.array_equal(pool.cpu().numpy()[:want.size], want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("codec", ["rans", "int8"])
+@pytest.mark.parametrize("D", [64, 96, 128])
+def test_scale_zero_pages_with_absent_tokens(codec, D):
+    """An absmax below 64 of the smallest denormals gives a scale of 0: present values become -128 (their quotients are
+    infinite or no number), absent tokens stay 0, whatever the page's token count leaves of the last four tokens."""
+    import torch
+    from chromofold_amd import kv
+    print(f"case {codec} D={D}", flush=True)
+    cdc = kv.CODEC_RANS_HYBRID if codec == "rans" else kv.CODEC_INT8
+    rng = np.random.default_rng(D)
+    tc = np.array([1, 2, 3, 4, 5, 7, 9, 11, 13, 14, 15, 16, 6, 10, 12, 8], np.uint32)
+    tiny = rng.integers(-63, 64, (16, 16, D)).astype(np.float64) * 2.0 ** -149
+    tiny[:, 0, 0] = 63 * 2.0 ** -149
+    V = tiny.astype(np.float32)
+    K = rng.standard_normal((16, 16, D)).astype(np.float32)
+    K[8:] = V[:8]
+    tables = np.concatenate([kv.build_table(rng.standard_normal((4, 16, D)).astype(np.float32)) for _ in range(2)])
+    tables = tables if codec == "rans" else None
+    first, counts = np.arange(0, 16, 4).astype(np.uint64), np.full(4, 4, np.uint32)
+    with np.errstate(all="ignore"):
+        want, offs = kv.encode_groups(cdc, K, V, D, tables, first, counts, None, tc)
+    up = lambda a, t=None: None if a is None else torch.from_numpy(a if t is None else a.astype(t)).to("cuda:0")  # noqa: E731
+    pool = torch.zeros(want.size + 4096, dtype=torch.uint8, device="cuda:0")
+    r = kv.encode_groups_device(cdc, up(K), up(V), D, up(tables), up(first, np.int64), up(counts, np.int32), pool, 0, None,
+                                up(tc, np.int32))
+    torch.cuda.synchronize()
+    assert int(r.status.item()) == 0 and int(r.pool_end.item()) == want.size
+    assert np.array_equal(r.offsets.cpu().numpy().view(np.uint32), offs)
+    assert np.array_equal(pool.cpu().numpy()[:want.size], want)
