@@ -156,10 +156,8 @@ __device__ __forceinline__ uint32_t offset_binary(uint32_t w) {
 // Four values of a page as a symbol word. The quotients are x * (1 / scale); where that may round to another integer
 // than the IEEE quotient x / scale (its error is below 3e-5 at quotients up to 128, so only within that distance of a
 // half), or is no number, the wavefront takes the exact division for the word (1.5 % of words). `exact` (wave-uniform):
-// the scale is so small or large that its reciprocal is not accurate. Values from `present` on are absent tokens' zeros,
-// whose symbol is 0 also where the scale is 0 (an absmax of a few denormals) and the quotient no number.
-__device__ __forceinline__ uint32_t quant_word(const float (&x)[4], float scale, float rscale, bool exact, bool rans,
-                                               uint32_t present = 4) {
+// the scale is so small or large that its reciprocal is not accurate.
+__device__ __forceinline__ uint32_t quant_word(const float (&x)[4], float scale, float rscale, bool exact, bool rans) {
   float r[4];
   bool doubt = exact;
 #pragma unroll
@@ -187,7 +185,7 @@ __device__ __forceinline__ uint32_t quant_word(const float (&x)[4], float scale,
   w = 0;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const uint32_t b = static_cast<uint32_t>(i) < present ? quant8(x[i], scale) : 128u;
+    const uint32_t b = quant8(x[i], scale);
     w |= (!rans ? b : b >= 128u ? b - 128u : b == 0u ? 128u : 256u - b) << (8 * i);
   }
   return w;
@@ -356,14 +354,25 @@ __global__ void __launch_bounds__(kEncThreads) encode_kernel(EncodeArgs a) {
             float x4[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i) x4[i] = static_cast<uint32_t>(4 * tq + i) < tc ? vx[r][4 * tq + i] : 0.0f;
-            w = quant_word(x4, vs, rvs, vx_exact, rans, tc - 4 * tq);
+            w = quant_word(x4, vs, rvs, vx_exact, rans);
             minus |= has_minus128(w, rans);
           }
           vT[X][(G * kMaxDim + d) * kVStride + tq] = w;
         }
       }
     }
-    if (__ballot(minus) != 0 && lane == 0) atomicOr(&s_minus[X], 1u);
+    if (__builtin_expect(__ballot(minus) != 0, 0)) {
+      if (lane == 0) atomicOr(&s_minus[X], 1u);
+      // a scale of 0 (an absmax of a few denormals) makes quotients of absent tokens NaN as well: their symbols are 0
+      if (__ballot(vs == 0.0f) != 0 && (tc & 3u) != 0u) {
+        const uint32_t keep = (1u << (8u * (tc & 3u))) - 1u;
+#pragma unroll 1
+        for (uint32_t d = lane; d < D; d += 64) {
+          uint32_t &w = vT[X][(G * kMaxDim + d) * kVStride + tc / 4];
+          w = (w & keep) | (absent & ~keep);
+        }
+      }
+    }
     if (lane == 0) {
       s_scale[X][0][G] = tc ? ks : 1.0f;
       s_scale[X][1][G] = tc ? vs : 1.0f;
