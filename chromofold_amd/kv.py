@@ -142,6 +142,20 @@ def encode_groups_device(codec: int, keys: torch.Tensor, values: torch.Tensor, h
     return DeviceEncodeResult(offs, end, status)
 
 
+def _give_workspace(d: cf_kv_batched_desc, nbytes: int, device: torch.device, stream) -> torch.Tensor:
+    """Points the descriptor at a workspace of its own, which it keeps alive (its fields hold only the address). The
+    memory is allocated on the stream whose calls use it, so that, let go of, it is reused behind them; inside a graph
+    capture it comes from the graph's memory."""
+    if device.type == "cuda" and stream != torch.cuda.current_stream(device):
+        with torch.cuda.stream(stream):
+            ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
+    else:
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
+    d.workspace_tensor, d.workspace_stream = ws, stream.cuda_stream
+    d.workspace, d.workspace_bytes = ws.data_ptr(), nbytes
+    return ws
+
+
 @dataclass
 class BatchedKv:
     """Device-resident pages of `seq_count` sequences x `kv_heads` heads for the batched decode entry point."""
@@ -157,9 +171,7 @@ class BatchedKv:
     host_pool: np.ndarray | None = None
     host_offsets: np.ndarray | None = None
     host_tables: np.ndarray | None = None
-    workspace: torch.Tensor | None = None
-    workspace_stream: int | None = None  # the stream whose calls use `workspace`; another stream has its own
-    stream_workspaces: dict = field(default_factory=dict)
+    workspace: torch.Tensor | None = None  # the latest descriptor's
     stats: dict = field(default_factory=dict)
 
     @property
@@ -168,8 +180,9 @@ class BatchedKv:
 
     def desc(self, queries: torch.Tensor, output: torch.Tensor, query_pos: torch.Tensor, softmax_scale: float,
              splits: int = 0, shared_groups: int = 0, stream=None) -> cf_kv_batched_desc:
-        """Descriptor (with a workspace of this object's for the stream, the current one by default) for attention();
-        shared_groups > 0 sizes the workspace for the cascade entry point."""
+        """Descriptor for attention(); shared_groups > 0 sizes the workspace for the cascade entry point. It holds a
+        workspace of its own (workspace_tensor), for calls on `stream` (the current one by default). Keep it as long as
+        a graph captured with it."""
         d = cf_kv_batched_desc()
         d.struct_size = C.sizeof(cf_kv_batched_desc)
         d.abi_version = EXT_ABI_VERSION
@@ -195,33 +208,23 @@ class BatchedKv:
         else:
             need = int(A.lib().cf_kv_batched_workspace_bytes(C.byref(d)))
         if need:
-            ws = self._stream_workspace(need, (stream if stream is not None else torch.cuda.current_stream()).cuda_stream)
-            d.workspace = ws.data_ptr()
-            d.workspace_bytes = ws.numel()
+            stream = stream if stream is not None else torch.cuda.current_stream()
+            self.workspace = _give_workspace(d, need, self.pool.device, stream)
         return d
-
-    def _stream_workspace(self, need: int, stream: int) -> torch.Tensor:
-        # calls on two streams may overlap, so each stream has a workspace of its own
-        if self.workspace is None or self.workspace_stream is None:
-            self.workspace_stream = stream
-        own = stream == self.workspace_stream
-        ws = self.workspace if own else self.stream_workspaces.get(stream)
-        if ws is None or ws.numel() < need:
-            ws = torch.empty(need, dtype=torch.uint8, device=self.pool.device)
-            if own:
-                self.workspace = ws
-            else:
-                self.stream_workspaces[stream] = ws
-        return ws
 
     def attention(self, queries: torch.Tensor, output: torch.Tensor, query_pos: torch.Tensor,
                   softmax_scale: float, splits: int = 0, stream=None, desc: cf_kv_batched_desc | None = None,
                   shared_groups: int = 0):
         """Batched decode; shared_groups > 0 uses the cascade entry point (the first shared_groups groups of every
-        sequence are sequence 0's, stored as INT8 blobs), with a descriptor made by desc(..., shared_groups=)."""
+        sequence are sequence 0's, stored as INT8 blobs), with a descriptor made by desc(..., shared_groups=). A
+        descriptor may be used on any stream."""
         stream = stream if stream is not None else torch.cuda.current_stream()
-        d = desc if desc is not None else self.desc(queries, output, query_pos, softmax_scale, splits, shared_groups, stream)
         s = stream.cuda_stream
+        d = desc if desc is not None else self.desc(queries, output, query_pos, softmax_scale, splits, shared_groups, stream)
+        if d.workspace and getattr(d, "workspace_stream", s) != s:
+            # made for another stream, whose calls may overlap this one: a copy with a workspace of this stream's
+            d = cf_kv_batched_desc.from_buffer_copy(d)
+            _give_workspace(d, d.workspace_bytes, self.pool.device, stream)
         if shared_groups:
             A.check(A.lib().cf_kv_paged_attention_cascade_async(C.byref(d), shared_groups, s),
                     "cf_kv_paged_attention_cascade_async")

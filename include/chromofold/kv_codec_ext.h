@@ -117,8 +117,9 @@ typedef struct cf_kv_group_header {
  *   queries      [seq_count, query_head_count, head_dim] fp32, output the same shape
  * A shared prefix is expressed by several sequences pointing at the same group blobs (refcounted pages).
  * `workspace` is caller-owned device memory of cf_kv_batched_workspace_bytes() bytes (span or split-context
- * partials; with splits = 0 a smaller one, or none, runs a launch that needs less where there is one);
- * the entry point allocates nothing and never synchronises. */
+ * partials; with splits = 0 a smaller one, or none, runs a launch that needs less where there is one). Calls that
+ * may overlap (two streams, a graph's replays beside eager calls) need a workspace each, whatever the shape.
+ * The entry point allocates nothing and never synchronises. */
 typedef struct cf_kv_batched_desc {
     uint32_t struct_size;
     uint32_t abi_version;
