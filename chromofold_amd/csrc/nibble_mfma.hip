@@ -226,8 +226,11 @@ __device__ void active_page(const AttnItem &it, const AttnShape &sh, uint32_t h,
         const float s = cfd::row16_sum(d) * it.scale_log2;
         if (!valid) continue;  // the whole row of lanes
         const float mn = fmaxf(m[j], s);
-        const float a = m[j] == kNegInf ? 0.0f : __builtin_amdgcn_exp2f(m[j] - mn), p = __builtin_amdgcn_exp2f(s - mn);
-        m[j] = mn;
+        const float a = m[j] == kNegInf ? 0.0f : __builtin_amdgcn_exp2f(m[j] - mn);
+        // a score of -inf (the tail's values are not checked) has no weight, also where the maximum is still -inf; one
+        // that is no number makes the row NaN, in a row of lanes (and a wavefront) that counts when states are merged
+        const float p = s == kNegInf ? 0.0f : __builtin_amdgcn_exp2f(s - mn);
+        m[j] = s == s ? mn : fmaxf(mn, -3.4e38f);
         l[j] = l[j] * a + (t == 0 ? p : 0.0f);
 #pragma unroll
         for (int e = 0; e < 8; ++e) acc[e][j] = fmaf(p, vf[e], acc[e][j] * a);
