@@ -45,6 +45,9 @@ constexpr uint32_t kRowBytes = kD / 2;                    // nibbles of one toke
 constexpr uint32_t kChunkStride = 16 * kRowBytes + 64;   // staged 16-row chunk + a bank offset between chunks
 constexpr uint32_t kTileBytes = 4 * kChunkStride;
 constexpr float kNegInf = -__builtin_huge_valf();
+constexpr float kLowest = -__FLT_MAX__;  // running maximum before the first token: below or equal to every finite score
+constexpr float kWeightTop = 32768.0f;                    // of a weight in the accumulators' unit
+constexpr int kUnitMax = 100;  // units 2^-100 to 2^100: V scales from 2^-85 (smaller ones lose bits) to 2^115
 
 __device__ inline half4_t as_half4(uint32_t lo, uint32_t hi) {
   half4_t h;
@@ -226,11 +229,10 @@ __device__ void active_page(const AttnItem &it, const AttnShape &sh, uint32_t h,
         const float s = cfd::row16_sum(d) * it.scale_log2;
         if (!valid) continue;  // the whole row of lanes
         const float mn = fmaxf(m[j], s);
-        const float a = m[j] == kNegInf ? 0.0f : __builtin_amdgcn_exp2f(m[j] - mn);
-        // a score of -inf (the tail's values are not checked) has no weight, also where the maximum is still -inf; one
-        // that is no number makes the row NaN, in a row of lanes (and a wavefront) that counts when states are merged
-        const float p = s == kNegInf ? 0.0f : __builtin_amdgcn_exp2f(s - mn);
-        m[j] = s == s ? mn : fmaxf(mn, -3.4e38f);
+        // the maximum is never -inf (kLowest): a score of -inf (the tail's values are not checked) has no weight, and
+        // one that is no number makes the row NaN, in a row of lanes that counts when states are merged
+        const float a = __builtin_amdgcn_exp2f(m[j] - mn), p = __builtin_amdgcn_exp2f(s - mn);
+        m[j] = mn;
         l[j] = l[j] * a + (t == 0 ? p : 0.0f);
 #pragma unroll
         for (int e = 0; e < 8; ++e) acc[e][j] = fmaf(p, vf[e], acc[e][j] * a);
@@ -282,11 +284,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
   float4_t acc[8];
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    m_run[j] = kNegInf;
+    m_run[j] = kLowest;
     l_run[j] = 0.0f;
   }
 #pragma unroll
   for (int e = 0; e < 8; ++e) acc[e] = float4_t{0, 0, 0, 0};
+  // acc is kept in units of 2^-vunit (one per 16-lane row), which the largest V scale met so far sets: f16 hi + lo holds
+  // a weight p * v_scale to 2^-25 of the unit, and in units of 1, with V scales around 0.3, that quantised small weights
+  // (relative error of an output row against float64, 26 items of 500-12000 tokens: 3.2e-7, in this unit 2.4e-7)
+  int vunit = kUnitMax;
+  float vfac = ldexpf(1.0f, vunit);
 
   // per-lane metadata of the tile in flight: this lane's token (row of chunk G), its visibility and scales
   bool n_ok = false;
@@ -428,7 +435,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
   // tiles, its loads share the wait for the first tile's copies. (A launch of its own for the tails took 14 us of a
   // batch and added partials to merge.)
   if (it.active_count != 0u && split + 1u == it.page_splits)
+  {
     active_page(it, sh, h, qt, qc, PG, wave, G, t, m_run, l_run, acc);
+    // into the unit of its own magnitude
+    float top = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) top = fmaxf(top, __builtin_fabsf(acc[e][j]));
+    top = cfd::row16_max(top);
+    if (top > 0.0f) vunit = min(max(15 - __builtin_amdgcn_frexp_expf(top), -kUnitMax), kUnitMax);
+    vfac = ldexpf(1.0f, vunit);
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[e][j] *= vfac;
+  }
 
   for (; tile < te; tile += kWaves) {
     // this tile's rows and scales and the next tile's descriptors have landed. K and V have one buffer each: the next
@@ -479,29 +501,45 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
       mx[j] = sc[j];
     }
     row_max4(mx);
-    // raise the running maxima (and rescale the accumulators) only when some lane's maximum grew
-    bool grow = false;
+    // V scales in the accumulators' unit: a weight p * v_scale * 2^vunit stays below 2^15
+    float vs[NB], vmax = 0.0f;
+#pragma unroll
+    for (int s = 0; s < NB; ++s) {
+      vs[s] = n_vs[s] * vfac;
+      vmax = fmaxf(vmax, vs[s]);
+    }
+    // raise the running maxima and the unit (and rescale the accumulators) only when some lane's grew
+    bool grow = vmax >= kWeightTop;
 #pragma unroll
     for (int j = 0; j < 4; ++j) grow |= mx[j] > m_run[j];
     if (__ballot(grow) != 0) {
+      float top = 0.0f;
+#pragma unroll
+      for (int s = 0; s < NB; ++s) top = fmaxf(top, n_vs[s]);
+      const int un = min(vunit, max(15 - __builtin_amdgcn_frexp_expf(cfd::row16_max(top)), -kUnitMax)), du = un - vunit;
+      vunit = un;
+      vfac = ldexpf(1.0f, un);
+#pragma unroll
+      for (int s = 0; s < NB; ++s) vs[s] = n_vs[s] * vfac;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const float mn = fmaxf(m_run[j], mx[j]);
-        const float alpha = (m_run[j] == kNegInf) ? 0.0f : __builtin_amdgcn_exp2f(m_run[j] - mn);
+        const float alpha = __builtin_amdgcn_exp2f(m_run[j] - mn);
         l_run[j] *= alpha;
+        const float beta = ldexpf(alpha, du);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) acc[e][j] *= alpha;
+        for (int e = 0; e < 8; ++e) acc[e][j] *= beta;
         m_run[j] = mn;
       }
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const float p = tok_ok ? __builtin_amdgcn_exp2f(sc[j] - m_run[j]) : 0.0f;
+      const float p = __builtin_amdgcn_exp2f(sc[j] - m_run[j]);  // 0 for a score of -inf
       l_run[j] += p;
       s_p[wave][j][lane] = p;
     }
 #pragma unroll
-    for (int s = 0; s < NB; ++s) s_vs[wave][s][lane] = n_vs[s];
+    for (int s = 0; s < NB; ++s) s_vs[wave][s][lane] = vs[s];
     wave_sync_lds();
 
     // ---- V: out[head][8t + e] += sum over 4 tokens of p * v_scale * (nibble - 8)
@@ -556,11 +594,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const float mw = cfd::rows4_max(m_run[j]);
-    const float f = (m_run[j] == kNegInf) ? 0.0f : __builtin_amdgcn_exp2f(m_run[j] - mw);
+    const float f = __builtin_amdgcn_exp2f(m_run[j] - mw);
+    const float g = ldexpf(f, -vunit);
     l_run[j] = cfd::rows4_sum(cfd::row16_sum(l_run[j] * f));
 #pragma unroll
-    for (int e = 0; e < 8; ++e) acc[e][j] = cfd::rows4_sum(acc[e][j] * f);
-    m_run[j] = mw;
+    for (int e = 0; e < 8; ++e) acc[e][j] = cfd::rows4_sum(acc[e][j] * g);
+    m_run[j] = l_run[j] == 0.0f ? kNegInf : mw;  // nothing seen
   }
   __syncthreads();  // every wave is done with its tile buffers: reuse them for the partials
   float(*red)[4][kD + 2] = reinterpret_cast<float(*)[4][kD + 2]>(&s_kv[0][0][0]);
