@@ -1437,26 +1437,27 @@ __global__ __launch_bounds__(kPfxThreads) __attribute__((amdgpu_waves_per_eu(2))
         }
       }
     }
-    // P V units: O is kept in units of 2^e_run with e_run >= (exponent of the group's largest present-page V scale)
-    // - 14, so the f16 operand p * v_scale * 2^-e_run stays below 2^15 whatever the V magnitude and weights down to
-    // 2^-25 of the running maximum stay normal
+    // P V units: O is kept in units of 2^e_run, e_run = (exponent of the group's largest present-page V scale) - 15, so
+    // that the f16 operand p * v_scale * 2^-e_run stays below 2^16 whatever the V magnitude (p <= 2; its hi part, rounded
+    // toward zero, stays finite) and weights down to 2^-29 of the reference stay normal. Units that follow the scales only
+    // every two binades, or 2^14 at the top, would skip more rescales but cost weights of 2^-18 and less their last bits
+    // (2^-24 of the largest: 3e-4 off instead of 1e-5), which shows where the heavy tokens have no V to speak of.
     float vscale[4], vmax = 0.0f;
 #pragma unroll
     for (int G = 0; G < 4; ++G) {
       vscale[G] = __uint_as_float(word(12 + G));
       if (((G < 2 ? tc01 : tc23) >> (16 * (G & 1)) & 0xFFFFu) != 0u) vmax = fmaxf(vmax, vscale[G]);
     }
-    const int ev = __builtin_amdgcn_readfirstlane(__builtin_amdgcn_frexp_expf(vmax)) - 14;
+    const int ev = __builtin_amdgcn_readfirstlane(__builtin_amdgcn_frexp_expf(vmax)) - 15;
     // Online softmax of row j over the group's 64 tokens. The reference m and the units move only when a row's
-    // maximum passes m by more than ln 2 (p stays <= 2) or the V exponent rises, or falls by more than 2: most groups
-    // then skip the rescale of O.
+    // maximum passes m by more than ln 2 (p stays <= 2) or the V exponent changes: other groups skip the rescale of O.
     float mx = -INFINITY;
 #pragma unroll
     for (int G = 0; G < 4; ++G)
 #pragma unroll
       for (int r = 0; r < 4; ++r) mx = fmaxf(mx, st[G][r]);
     mx = cfd::rows4_max(mx);
-    if (__ballot(mx > m + 0.6931f) || ev > e_run || ev < e_run - 2) {
+    if (__ballot(mx > m + 0.6931f) || ev != e_run) {
       const float mn = fmaxf(m, mx);
       const float alpha = m == -INFINITY ? 0.0f : __expf(m - mn);
       m = mn;
