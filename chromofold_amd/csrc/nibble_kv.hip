@@ -247,13 +247,15 @@ template <int LG, int G>
 __global__ __launch_bounds__(256) void nib_attn_kernel(const AttnItem *__restrict__ items, WorkList work, AttnShape sh,
                                                        uint32_t hw, uint32_t hgroups, uint32_t qchunks,
                                                        float *__restrict__ ws) {
-  const uint32_t ii = work_item(work.first, work.items, blockIdx.x);
+  const uint32_t block = work_block();
+  if (block >= work.total) return;
+  const uint32_t ii = work_item(work.first, work.items, block);
   const AttnItem &it = items[ii];
   // splits [0, vbase) are the MFMA kernel's (which takes its items' active pages along), then vsplits page splits of
   // this kernel, then asplits over the active page; an item with nothing visible has one (empty) split
   const uint32_t vbase = it.mfma_nb ? it.page_splits : 0u;
   const uint32_t mine_n = it.nsplit - vbase;  // this kernel's splits of the item (at least 1 where it owns units)
-  const uint32_t local = blockIdx.x - work.first[ii];
+  const uint32_t local = block - work.first[ii];
   const uint32_t y = local / mine_n, split = vbase + (local - y * mine_n);
   const uint32_t per_tok = hgroups * qchunks;
   const uint32_t qt = y / per_tok;
@@ -438,7 +440,7 @@ __global__ __launch_bounds__(256) void nib_attn_kernel(const AttnItem *__restric
 constexpr uint32_t kMergeRows = 4;  // rows (waves) per workgroup
 __global__ __launch_bounds__(64 * kMergeRows) void nib_merge_kernel(const AttnItem *__restrict__ items, WorkList work,
                                                                     AttnShape sh, const float *__restrict__ ws) {
-  const uint32_t unit = __builtin_amdgcn_readfirstlane(blockIdx.x * kMergeRows + (threadIdx.x >> 6));
+  const uint32_t unit = __builtin_amdgcn_readfirstlane(work_block() * kMergeRows + (threadIdx.x >> 6));
   if (unit >= work.total) return;
   const uint32_t ii = work_item(work.first, work.items, unit);
   const AttnItem &it = items[ii];
@@ -499,7 +501,7 @@ __global__ __launch_bounds__(64 * kMergeRows) void nib_merge_kernel(const AttnIt
 template <int LG, int G>
 hipError_t launch_attn_lg_g(const WorkList &work, dim3 block, hipStream_t s, const AttnItem *items,
                             const AttnShape &sh, uint32_t hw, uint32_t hgroups, uint32_t qchunks, float *ws) {
-  nib_attn_kernel<LG, G><<<work.total, block, 0, s>>>(items, work, sh, hw, hgroups, qchunks, ws);
+  nib_attn_kernel<LG, G><<<work_grid(work.total), block, 0, s>>>(items, work, sh, hw, hgroups, qchunks, ws);
   return hipPeekAtLastError();
 }
 
@@ -591,7 +593,7 @@ hipError_t AttnRunner::run(const std::vector<AttnRequest> &reqs, const AttnShape
 
   std::vector<AttnItem> items(reqs.size());
   uint64_t floats = 0;
-  uint32_t max_split = 1, max_qtok = 1;
+  uint32_t max_qtok = 1;
   bool any_nb[5] = {false, false, false, false, false};
   const uint32_t wave_lanes = std::min(64u, hw * lg);  // lanes of the VALU kernel's first wave
   for (size_t i = 0; i < reqs.size(); ++i) {
@@ -644,11 +646,10 @@ hipError_t AttnRunner::run(const std::vector<AttnRequest> &reqs, const AttnShape
     if (it.nsplit == 0u) it.nsplit = 1u;  // nothing visible: one empty split, the row comes out 0
     it.ws_offset = floats;
     floats += uint64_t(it.nsplit) * it.q_tokens * sh.q_heads * (D + 4u);
-    max_split = std::max(max_split, it.nsplit);
     max_qtok = std::max(max_qtok, it.q_tokens);
   }
-  const uint64_t ydim = uint64_t(max_qtok) * hgroups * qchunks;
-  if (ydim > 65535u || reqs.size() > 65535u || max_split > 0x7fffffffu) {
+  // the size of one call, which callers know by this error (the launches themselves hold 2^31 workgroups, checked below)
+  if (uint64_t(max_qtok) * hgroups * qchunks > 65535u || reqs.size() > 65535u) {
     error = "attention batch exceeds the launch grid (too many query tokens or items in one call)";
     return hipErrorInvalidValue;
   }
@@ -667,7 +668,7 @@ hipError_t AttnRunner::run(const std::vector<AttnRequest> &reqs, const AttnShape
     uint32_t *first = reinterpret_cast<uint32_t *>(table.data() + list_at) + l * (n + 1);
     uint64_t at = 0;
     for (size_t i = 0; i <= n; ++i) {
-      if (at > 0x7fffffffu) {
+      if ((l < 2 ? at : (at + 7u) / 8u * 8u * sh.kv_heads) > 0x7fffffffu) {  // (MFMA units are workgroups per KV head)
         error = "attention batch exceeds the launch grid (too many query tokens or items in one call)";
         return hipErrorInvalidValue;
       }
@@ -722,7 +723,7 @@ hipError_t AttnRunner::run(const std::vector<AttnRequest> &reqs, const AttnShape
     if (e != hipSuccess) return e;
   }
   if (totals[1])
-    nib_merge_kernel<<<(totals[1] + kMergeRows - 1u) / kMergeRows, 64 * kMergeRows, 0, stream>>>(d_items, work(1), sh,
+    nib_merge_kernel<<<work_grid((totals[1] + kMergeRows - 1u) / kMergeRows), 64 * kMergeRows, 0, stream>>>(d_items, work(1), sh,
                                                                                                  partials);
   e = hipPeekAtLastError();
   if (e == hipSuccess) launches_ = 2;

@@ -259,7 +259,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
   // heads lie side by side, 64 bytes each, its scales 16 bytes each), so the heads of a unit are 8 workgroups apart:
   // one XCD's L2, close in time. (Heads across XCDs fetched 1.5x the bytes at 32 sequences of 32768 tokens.)
   const uint32_t kvh = sh.kv_heads, gqa = sh.gqa;
-  const uint32_t oct = blockIdx.x / (8u * kvh), in_oct = blockIdx.x - oct * (8u * kvh);
+  const uint32_t block = work_block(), oct = block / (8u * kvh), in_oct = block - oct * (8u * kvh);
   const uint32_t unit = 8u * oct + (in_oct & 7u), h = in_oct >> 3;
   if (unit >= work.total) return;
   const uint32_t ii = work_item(work.first, work.items, unit);
@@ -653,7 +653,7 @@ hipError_t launch_nib_mfma(uint32_t nb, const AttnItem *items, const WorkList &w
   const uint32_t qchunks = (sh.gqa + 3u) / 4u;
   const uint64_t blocks = (uint64_t(work.total) + 7u) / 8u * 8u * sh.kv_heads;
   if (blocks > 0x7fffffffu) return hipErrorInvalidValue;
-  const dim3 grid(static_cast<uint32_t>(blocks));
+  const dim3 grid = work_grid(blocks);
   switch (nb) {
     case 1: nib_mfma_kernel<1><<<grid, 256, 0, stream>>>(items, work, sh, qchunks, ws); break;
     case 2: nib_mfma_kernel<2><<<grid, 256, 0, stream>>>(items, work, sh, qchunks, ws); break;

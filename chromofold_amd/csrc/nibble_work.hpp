@@ -15,6 +15,15 @@
 
 namespace cfnib {
 
+// Grid of `blocks` workgroups (at most 2^31) of up to 256 threads: a dimension of a launch holds 2^32 work-items, so
+// larger grids go on in y, kGridX (a multiple of the 8 XCDs, which take consecutive workgroups in turn) to a row.
+constexpr uint32_t kGridX = 1u << 22;
+inline dim3 work_grid(uint64_t blocks) {
+  if (blocks <= kGridX) return dim3(static_cast<uint32_t>(blocks));
+  return dim3(kGridX, static_cast<uint32_t>((blocks + kGridX - 1u) / kGridX));
+}
+__device__ __forceinline__ uint32_t work_block() { return blockIdx.y * kGridX + blockIdx.x; }  // may be past the last
+
 // The item that owns unit `u` (u < first[items]): the last i with first[i] <= u, which skips items without units.
 __device__ __forceinline__ uint32_t work_item(const uint32_t *__restrict__ first, uint32_t items, uint32_t u) {
   uint32_t lo = 0, hi = items;  // first[lo] <= u < first[hi]
