@@ -437,7 +437,7 @@ __device__ __forceinline__ void wide_block(uint32_t w, uint32_t np, uint32_t &lo
 // has `nwg` wide workgroups per KV head (one per CU in all) and lays the head's chain pairs of all sequences end to
 // end: P pairs, sequence s the pairs [pre[s], pre[s + 1]). Workgroup j takes the pairs [j P / nwg, (j + 1) P / nwg),
 // its wavefronts blocks of them (wide_block), whatever sequences they fall in; the rANS tables are staged once per
-// workgroup. 48 sequences of 150-8000 tokens: 116 us with splits of the longest, see kv_batched_kernel.
+// workgroup. 48 sequences of 150-8000 tokens: 104 us with splits of the longest, 55 us as spans (see BatchedPlan).
 // A wavefront's block is a run of segments, one per sequence it touches. Every segment but its last ends where the
 // sequence ends, so it is the only such segment of that sequence: its state goes to slot nwaves + s. Last segments go
 // to the wavefront's slot, those of consecutive wavefronts of a workgroup that lie in one sequence merged into the
@@ -891,19 +891,18 @@ __global__ CF_KV_OCC __launch_bounds__(64 * kWavesWide) void kv_span_kernel(cf_k
   struct Cur {
     uint32_t s, g, end;
   };
+  auto uni = [](uint32_t v) { return static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(v)); };
   auto enter = [&](uint32_t s, uint32_t x) {  // the groups of sequence s from its pair at x on, inside [x0, x1)
-    const uint32_t a = s_pre[s], b = s_pre[s + 1];
-    const uint32_t vis = s_vis[s];
-    const uint32_t own = (vis + 63u) / 64u, stop = 2u * (min(b, s_wave[wave][2]) - a);
+    const uint32_t a = uni(s_pre[s]), b = uni(s_pre[s + 1]), vis = uni(s_vis[s]);
+    const uint32_t own = (vis + 63u) / 64u, stop = 2u * (min(b, uni(s_wave[wave][2])) - a);
     return Cur{s, 2u * (x - a), static_cast<uint32_t>(min(min(own, d.max_groups), stop))};
   };
-  auto advance = [&](Cur c) {
-    if (c.s == kNoSeq) return c;
+  auto advance = [&](Cur c) {  // c: wave-uniform, not past the end
     if (c.g + 1 < c.end) return Cur{c.s, c.g + 1, c.end};
-    const uint32_t x = s_pre[c.s + 1];  // the next pair of the head's list
-    if (x >= s_wave[wave][2]) return Cur{kNoSeq, 0, 0};
+    const uint32_t x = uni(s_pre[c.s + 1]);  // the next pair of the head's list
+    if (x >= uni(s_wave[wave][2])) return Cur{kNoSeq, 0, 0};
     uint32_t s = c.s + 1;
-    while (s_pre[s + 1] == x) ++s;  // sequences without own groups
+    while (uni(s_pre[s + 1]) == x) ++s;  // sequences without own groups
     return enter(s, x);
   };
   Cur cur{kNoSeq, 0, 0};
@@ -914,8 +913,9 @@ __global__ CF_KV_OCC __launch_bounds__(64 * kWavesWide) void kv_span_kernel(cf_k
     const uint32_t n = static_cast<uint32_t>(__builtin_popcountll(__builtin_amdgcn_ballot_w64(lane < 12 && k2 < S && s_pre[min(k2, S)] <= x0)));
     cur = enter(c + n - 1u, x0);
   }
-  // Wave-uniform, but not to be seen as such: with a loop that the compiler knows to be uniform it schedules the decode
-  // for 216 VGPRs and spills 49.
+  // Wave-uniform, but the loop is not to be seen as such: with one that the compiler knows to be uniform it schedules the
+  // decode for 216 VGPRs and spills 49. Inside the loop they are made scalars again: conditions and addresses in vector
+  // registers cost 60 VALU and 50 SALU instructions a group, 6 % of the loop.
   asm volatile("" : "+v"(cur.s), "+v"(cur.g), "+v"(cur.end));
 
   constexpr int NC = NQ / 16 > 0 ? NQ / 16 : 1;
@@ -970,9 +970,14 @@ __global__ CF_KV_OCC __launch_bounds__(64 * kWavesWide) void kv_span_kernel(cf_k
   auto offset_of = [&](const Cur &c) {
     return d.group_offsets[(static_cast<size_t>(c.s) * d.kv_head_count + head) * d.max_groups + c.g];
   };
-  Cur nxt = advance(cur);
+  Cur nxt{kNoSeq, 0, 0};
+  if (x0 < x1) nxt = advance(Cur{uni(cur.s), uni(cur.g), uni(cur.end)});
   uint32_t off_next = nxt.s != kNoSeq ? offset_of(nxt) : 0u;
-  const uint8_t *blob = cur.s != kNoSeq ? d.pool + static_cast<size_t>(offset_of(cur)) * 16 : d.pool;
+  // (a scalar address: in vector registers it costs the loads' addresses more of them and 3-5 % of the loop)
+  auto blob_at = [&](uint32_t off) {
+    return d.pool + static_cast<size_t>(static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(off))) * 16;
+  };
+  uint32_t off_cur = cur.s != kNoSeq ? offset_of(cur) : 0u;
   uint32_t h_cnt = 0, h_chain = 0, h_tc = 0, h_codec = 0;
   uint32_t h_st[2] = {0, 0};
   float h_ks = 0.f, h_vs = 0.f;
@@ -980,8 +985,9 @@ __global__ CF_KV_OCC __launch_bounds__(64 * kWavesWide) void kv_span_kernel(cf_k
     h_st[0] = reinterpret_cast<const uint32_t *>(b + kHdr)[lane];
     h_st[1] = reinterpret_cast<const uint32_t *>(b + kHdr)[64 + lane];
     h_cnt = *reinterpret_cast<const uint32_t *>(b + 4);
-    h_chain = *reinterpret_cast<const uint16_t *>(b + 8);
-    h_tc = reinterpret_cast<const uint16_t *>(b + 12)[G];
+    // (whole words, cut where they are used: halves cost 0.5 of 22.8 us at 40 x 4096 tokens, hd 64, INT8)
+    h_chain = *reinterpret_cast<const uint32_t *>(b + 8);
+    h_tc = reinterpret_cast<const uint32_t *>(b + 12)[G >> 1];
     h_ks = reinterpret_cast<const float *>(b + 32)[G];
     h_vs = reinterpret_cast<const float *>(b + 48)[G];
     h_codec = *reinterpret_cast<const uint32_t *>(b);
@@ -1004,27 +1010,32 @@ __global__ CF_KV_OCC __launch_bounds__(64 * kWavesWide) void kv_span_kernel(cf_k
   for (int w = 0; w < 14; ++w) pre[w] = 0;
   uint32_t vis_cur = 0;
   if (cur.s != kNoSeq) {
+    const uint8_t *blob = blob_at(off_cur);
     load_header(blob);
     load_queries(cur.s);
     vis_cur = s_vis[cur.s];
     if (RANS && h_codec == CF_KV_CODEC_RANS_HYBRID) {
-      const uint32_t *lw = raw_of(blob, h_chain);
+      const uint32_t *lw = raw_of(blob, h_chain & 0xFFFFu);
 #pragma unroll
       for (int w = 0; w < 7; ++w) {
         pre[w] = lw[w * 64 + lane];
         pre[7 + w] = lw[RAW + w * 64 + lane];
       }
-      stage_words(blob, h_chain, h_cnt);
+      stage_words(blob, h_chain & 0xFFFFu, h_cnt);
     }
   }
   uint32_t st[2] = {0, 0};
   bool broken = false, fresh = true;  // fresh: the segment's first group (a chain cannot continue into it)
-  const bool work = cur.s != kNoSeq;
+  const bool work = x0 < x1;
+  uint32_t seq_last = kNoSeq;
   while (cur.s != kNoSeq) {
-    const uint32_t cnt = h_cnt, chain = h_chain, tcG = h_tc, gcodec = h_codec;
+    // (the loop's own variables stay in vector registers, see above; inside they are scalars)
+    const uint32_t cs = uni(cur.s), cg = uni(cur.g);
+    const Cur nc{uni(nxt.s), uni(nxt.g), uni(nxt.end)};
+    const uint32_t cnt = h_cnt, chain = h_chain & 0xFFFFu, tcG = h_tc >> (16 * (G & 1)) & 0xFFFFu, gcodec = h_codec;
     const float ks = h_ks, vs = h_vs;
-    const uint8_t *curb = blob;
-    const bool tok_ok = static_cast<uint32_t>(t) < tcG && 64 * cur.g + 16 * G + t < vis_cur;
+    const uint8_t *curb = blob_at(off_cur), *blob = blob_at(off_next);
+    const bool tok_ok = static_cast<uint32_t>(t) < tcG && 64 * cg + 16 * G + t < vis_cur;
     if constexpr (RANS) {  // this group's copies (started during the previous group) have landed
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -1039,17 +1050,16 @@ __global__ CF_KV_OCC __launch_bounds__(64 * kWavesWide) void kv_span_kernel(cf_k
         broken |= fresh;
       }
     }
-    const Cur nc = nxt;
     if (nc.s != kNoSeq) {  // next group's header and states (its offset was loaded one group earlier)
-      blob = d.pool + static_cast<size_t>(off_next) * 16;
+      off_cur = off_next;
       load_header(blob);
       nxt = advance(nc);
       off_next = nxt.s != kNoSeq ? offset_of(nxt) : 0u;
     }
     const bool next_rans = RANS && nc.s != kNoSeq && h_codec == CF_KV_CODEC_RANS_HYBRID;
-    const uint32_t *nlw = next_rans ? raw_of(blob, h_chain) : nullptr;
+    const uint32_t *nlw = next_rans ? raw_of(blob, h_chain & 0xFFFFu) : nullptr;
     auto stage_next = [&]() {
-      if (next_rans) stage_words(blob, h_chain, h_cnt);
+      if (next_rans) stage_words(blob, h_chain & 0xFFFFu, h_cnt);
     };
     if (RANS && gcodec == CF_KV_CODEC_RANS_HYBRID) {
       group_body<D, CF_KV_CODEC_RANS_HYBRID, KL>(stage_next, pre, nlw, st, raw_of(curb, chain),
@@ -1061,53 +1071,51 @@ __global__ CF_KV_OCC __launch_bounds__(64 * kWavesWide) void kv_span_kernel(cf_k
           0, s_tab, qhi, qlo, qsum, s_p[wave], vl, lane, tok_ok, ks, vs, e_run, m_run, l_run, acc_v);
     }
     fresh = false;
-    if (nc.s != cur.s) {
-      if (nc.s == kNoSeq) break;  // the block's last segment: merged below
-      {
-        // ---- the sequence ends here and the block goes on: flush its state from registers (the word buffer is being
-        // filled for the next group). Row G of the lanes writes head G.
-        const uint32_t a = s_pre[cur.s];
-        const bool whole = a >= s_wave[wave][1];
-        float l4[kGqa], lg = 0.0f, mg = 0.0f, ag[D / 16];
+    if (nc.s != cs && nc.s != kNoSeq) {
+      // ---- the sequence ends here and the block goes on: flush its state from registers (the word buffer is being
+      // filled for the next group). Row G of the lanes writes head G.
+      const uint32_t a = s_pre[cs];
+      const bool whole = a >= s_wave[wave][1];
+      float l4[kGqa], lg = 0.0f, mg = 0.0f, ag[D / 16];
 #pragma unroll
-        for (int h = 0; h < kGqa; ++h) l4[h] = cfd::rows4_sum(cfd::row16_sum(l_run[h]));
+      for (int h = 0; h < kGqa; ++h) l4[h] = cfd::rows4_sum(cfd::row16_sum(l_run[h]));
+#pragma unroll
+      for (int h = 0; h < kGqa; ++h) {
+        lg = G == h ? l4[h] : lg;
+        mg = G == h ? m_run[h] : mg;
+      }
+      if (broken) mg = __builtin_nanf("");
+#pragma unroll
+      for (int i = 0; i < D / 16; ++i) {
+        ag[i] = 0.0f;
 #pragma unroll
         for (int h = 0; h < kGqa; ++h) {
-          lg = G == h ? l4[h] : lg;
-          mg = G == h ? m_run[h] : mg;
+          const float v = cfd::rows4_sum(G < 2 ? ldexpf(acc_v[i][h], e_run) : 0.0f);
+          ag[i] = G == h ? v : ag[i];
         }
-        if (broken) mg = __builtin_nanf("");
-#pragma unroll
-        for (int i = 0; i < D / 16; ++i) {
-          ag[i] = 0.0f;
-#pragma unroll
-          for (int h = 0; h < kGqa; ++h) {
-            const float v = cfd::rows4_sum(G < 2 ? ldexpf(acc_v[i][h], e_run) : 0.0f);
-            ag[i] = G == h ? v : ag[i];
-          }
-        }
-        if (whole) {
-          if (static_cast<uint32_t>(G) < gqa) {
-            float *o = d.output + (static_cast<size_t>(cur.s) * d.query_head_count + head * gqa + G) * D + t;
-#pragma unroll
-            for (int i = 0; i < D / 16; ++i) o[16 * i] = mg != mg ? mg : lg > 0.0f ? ag[i] / lg : 0.0f;
-          }
-        } else {
-          float *pp = head_slots + (static_cast<size_t>(sp.nwg) * W + cur.s) * (kGqa * (D + 2)) + G * (D + 2);
-#pragma unroll
-          for (int i = 0; i < D / 16; ++i) pp[16 * i + t] = ag[i];
-          if (t == 0) {
-            pp[D] = mg;
-            pp[D + 1] = lg;
-          }
-        }
-        reset();
-        broken = false;
-        fresh = true;
-        load_queries(nc.s);
-        vis_cur = s_vis[nc.s];
       }
+      if (whole) {
+        if (static_cast<uint32_t>(G) < gqa) {
+          float *o = d.output + (static_cast<size_t>(cs) * d.query_head_count + head * gqa + G) * D + t;
+#pragma unroll
+          for (int i = 0; i < D / 16; ++i) o[16 * i] = mg != mg ? mg : lg > 0.0f ? ag[i] / lg : 0.0f;
+        }
+      } else {
+        float *pp = head_slots + (static_cast<size_t>(sp.nwg) * W + cs) * (kGqa * (D + 2)) + G * (D + 2);
+#pragma unroll
+        for (int i = 0; i < D / 16; ++i) pp[16 * i + t] = ag[i];
+        if (t == 0) {
+          pp[D] = mg;
+          pp[D + 1] = lg;
+        }
+      }
+      reset();
+      broken = false;
+      fresh = true;
+      load_queries(nc.s);
+      vis_cur = s_vis[nc.s];
     }
+    seq_last = cs;
     cur = nc;
   }
 
@@ -1130,43 +1138,52 @@ __global__ CF_KV_OCC __launch_bounds__(64 * kWavesWide) void kv_span_kernel(cf_k
       }
     }
   }
-  if (lane == 0) s_wave[wave][0] = work ? cur.s : kNoSeq;
+  if (lane == 0) s_wave[wave][0] = seq_last;
   __syncthreads();
-  uint32_t leaders = 0;  // wavefronts that begin a run of equal sequences
+  // wavefronts that begin a run of equal sequences, and the end of the last run (idle wavefronts are the last ones)
+  uint32_t leaders = 0, last = 0;
+  {
+    uint32_t q[W];
 #pragma unroll
-  for (int w = 0; w < W; ++w) {
-    const uint32_t q = s_wave[w][0];
-    if (q != kNoSeq && (w == 0 || s_wave[w - 1][0] != q)) leaders |= 1u << w;
+    for (int w = 0; w < W; ++w) q[w] = s_wave[w][0];
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+      if (q[w] != kNoSeq && (w == 0 || q[w - 1] != q[w])) leaders |= 1u << w;
+      last = q[w] != kNoSeq ? w + 1 : last;
+    }
   }
   const uint32_t runs = static_cast<uint32_t>(__builtin_popcount(leaders));
   for (uint32_t i = threadIdx.x; i < runs * (kGqa * D); i += kThreads) {
     const uint32_t r = i / (kGqa * D), rest = i % (kGqa * D);
     uint32_t left = leaders;
     for (uint32_t k = 0; k < r; ++k) left &= left - 1;
-    const int w0 = __builtin_ctz(left);
+    const uint32_t w0 = static_cast<uint32_t>(__builtin_ctz(left));
     left &= left - 1;
-    const int w1 = left ? __builtin_ctz(left) : W;  // wavefronts past the run hold no sequence or another one
-    const uint32_t q = s_wave[w0][0];
+    const uint32_t w1 = left ? static_cast<uint32_t>(__builtin_ctz(left)) : last;  // the run is [w0, w1)
+    const uint32_t q = s_wave[w0][0], end = s_wave[w1 - 1][2];
     const int h = rest / D, dd = rest % D;
-    float m = -INFINITY;
+    // all wavefronts' values in flight together, those of the run used in ascending order (a loop over the run, whose
+    // every step waits for LDS, took 4 us)
+    float mw[W], m = -INFINITY;
     bool nan = false;
-    uint32_t end = 0;
-    for (int w = w0; w < w1 && s_wave[w][0] == q; ++w) {
-      const float mw = reinterpret_cast<const float *>(s_buf[w])[h * (D + 2) + D];
-      nan |= mw != mw;
-      m = fmaxf(m, mw);
-      end = s_wave[w][2];
+#pragma unroll
+    for (uint32_t w = 0; w < W; ++w) mw[w] = reinterpret_cast<const float *>(s_buf[w])[h * (D + 2) + D];
+#pragma unroll
+    for (uint32_t w = 0; w < W; ++w) {
+      if (w < w0 || w >= w1) mw[w] = -INFINITY;
+      nan |= mw[w] != mw[w];
+      m = fmaxf(m, mw[w]);
     }
     float l = 0.0f, o = 0.0f;
-    if (m != -INFINITY)
-      for (int w = w0; w < w1 && s_wave[w][0] == q; ++w) {
-        const float *rw = reinterpret_cast<const float *>(s_buf[w]);
-        const float mw = rw[h * (D + 2) + D];
-        if (mw == -INFINITY || mw != mw) continue;
-        const float sc = __expf(mw - m);
-        l += rw[h * (D + 2) + D + 1] * sc;
-        o += rw[h * (D + 2) + dd] * sc;
-      }
+#pragma unroll
+    for (uint32_t w = 0; w < W; ++w) {
+      const float *rw = reinterpret_cast<const float *>(s_buf[w]);
+      const float lw = rw[h * (D + 2) + D + 1], ow = rw[h * (D + 2) + dd];
+      if (mw[w] == -INFINITY || mw[w] != mw[w]) continue;
+      const float sc = __expf(mw[w] - m);
+      l += lw * sc;
+      o += ow * sc;
+    }
     if (nan) m = __builtin_nanf("");
     if (s_wave[w0][1] <= s_pre[q] && end >= s_pre[q + 1]) {  // the whole sequence
       if (static_cast<uint32_t>(h) < gqa)
@@ -1196,6 +1213,8 @@ __global__ __launch_bounds__(kGqa * D) void kv_span_merge_kernel(cf_kv_batched_d
   uint32_t n = 0;
   if (a < b) {  // one state per workgroup the sequence touches, then its own slot
     const uint32_t j0 = span_owner(a, P, sp.nwg), j1 = span_owner(b - 1, P, sp.nwg);
+    // one workgroup's whole range: one state, written by the span kernel (as in a batch of equal lengths)
+    if (j0 == j1 && span_begin(j0, P, sp.nwg) == a && span_begin(j0 + 1, P, sp.nwg) == b) return;
     n = j1 - j0 + 1;
     for (uint32_t k = threadIdx.x; k <= n; k += kGqa * D) s_slot[k] = kNone;
     __syncthreads();
@@ -2026,18 +2045,23 @@ uint32_t cu_count() {
 // second round leaves most CUs idle at the tail), keeping at least one page group per wavefront. A caller's d->splits
 // is kept.
 // Spans: batches of several sequences with fewer units than three per CU run as a span launch and its merge, which is
-// balanced whatever the lengths (the shapes above split every sequence the same way, as the host cannot see them): 116
-// -> 67 us for 48 sequences of 150-8000 tokens, 8 KV heads; 29.5 -> 20.2 us for 40 of 200-6000, 4 KV heads, hd 64, INT8.
-// Not for
+// balanced whatever the lengths (the shapes above split every sequence the same way, as the host cannot see them). Both
+// launches of the same library, us (8 KV / 32 query heads, hd 128, rANS, unless said otherwise):
+//                                    spans  splits                                     spans  splits
+//   48 x 150-8000 tokens              55.4   103.8     48 x 4096                        86.9    84.3
+//   32 x 500-32768                   111.0   298.9     32 x 32768                      378.3   375.9
+//   32 x 28000-32768                 355.2   361.5     32 x 8192                       105.8   103.5
+//   4 x 4000-131072                  101.1   148.3     4 x 131072                      198.2   195.8
+//   32 x 100-4096                     30.6    43.3     32 x 4096                        49.7    47.0
+//   40 x 200-6000, 4/8 heads,                          40 x 4096, 4/8 heads,
+//     hd 64, INT8                     18.1    23.5       hd 64, INT8                    23.9    22.8
+//   24 x 32768 (192 units, 256 CUs)  296.5   322.5     32 x 32768, INT8                321.0   315.8
+// A batch padded to one length pays 1.5-5 us (prologue and merge; the loops are alike), one whose mean is below 0.97 of
+// its longest (0.94 at 32 x 4096) gains. Not for
 //   * a single sequence, which cannot be ragged: the splits' smaller workgroups start sooner (17.3 against 24 us at 2003
 //     tokens);
-//   * contexts that the splits leave with less than two chain pairs per wavefront: there is little to balance, and the
-//     span launch's longer prologue and its merge cost 5 us (20 x 2000 tokens: 27.8 against 32.4 us, 4 x 300: 13.8
-//     against 20.2);
-//   * the one-split wide shape from kSpanMaxPairs pairs per wavefront up: it needs no merge, and a batch padded to one
-//     length loses the merge and the longer prologue to a span launch (32 x 32768 tokens: 397 against 405 us; at 32 x
-//     4096, 2.7 pairs per wavefront, 52.4 against 55.5 us padded to one length but 48.1 against 27.6 us ragged from 100
-//     tokens);
+//   * tables with room for so few groups that the splits leave less than two chain pairs per wavefront: there is little
+//     to balance, and prologue and merge cost 3 us (20 x 2000 tokens: 26.9 against 29.6 us, 32 x 300: 15.0 against 18.4);
 //   * larger grids: one workgroup per unit, which the dispatcher balances and whose neighbours share a common prefix in
 //     L1;
 //   * callers who fix the splits, or whose workspace is too small for the span states.
@@ -2045,7 +2069,7 @@ struct BatchedPlan {
   uint32_t splits, waves;
   uint32_t span_wg;  // > 0: a span launch with that many workgroups per KV head
 };
-constexpr uint32_t kWidePairsPerWave = 2, kSpanMaxPairs = 16;
+constexpr uint32_t kWidePairsPerWave = 2;
 
 BatchedPlan split_plan(const cf_kv_batched_desc *d) {
   const uint32_t units = d->seq_count * d->kv_head_count;
@@ -2073,7 +2097,7 @@ BatchedPlan batched_plan(const cf_kv_batched_desc *d) {
       static_cast<uint64_t>(d->seq_count) * d->kv_head_count >= 3u * cu_count())
     return p;
   const uint32_t pairs = (d->max_groups + 1) / 2, lanes = p.splits * p.waves;  // wavefronts of the longest context
-  if (pairs < 2 * lanes || (p.waves == 12u && p.splits == 1u && pairs >= kSpanMaxPairs * lanes)) return p;
+  if (pairs < 2 * lanes) return p;
   return {1u, 12u, span_workgroups(d->kv_head_count)};
 }
 

@@ -119,6 +119,9 @@ typedef struct cf_kv_group_header {
  * `workspace` is caller-owned device memory of cf_kv_batched_workspace_bytes() bytes (span or split-context
  * partials; with splits = 0 a smaller one, or none, runs a launch that needs less where there is one). Calls that
  * may overlap (two streams, a graph's replays beside eager calls) need a workspace each, whatever the shape.
+ * Results repeat bit for bit for the same descriptor contents and lengths. With splits = 0 the launch balances the batch
+ * over the chip by the sequences' lengths, so that a row's fp32 rounding depends on the lengths of the others in the
+ * batch (differences of about 1e-6 of a row); with splits given it depends on its own sequence alone.
  * The entry point allocates nothing and never synchronises. */
 typedef struct cf_kv_batched_desc {
     uint32_t struct_size;
@@ -153,13 +156,15 @@ cf_status cf_kv_validate_batched_desc(const cf_kv_batched_desc *desc);
  * semantics of one (sequence, query head) equal cf_kv_paged_attention_async with one query row and no tail. */
 cf_status cf_kv_paged_attention_batched_async(const cf_kv_batched_desc *desc, void *stream);
 
-/* Allocation-free variant of cf_kv_paged_attention_batched_async: the same launches and results, but the split
- * partials go to a library-owned device array of CF_KV_BATCHED_NOALLOC_SCRATCH_BYTES per GPU instead of
- * desc->workspace (ignored). No counterpart in the reference; it is for callers that cannot allocate device memory
- * (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc). It calls no allocator. A
- * descriptor whose split partials exceed that size returns CF_ERR_UNSUPPORTED (use the workspace entry point, or
- * fewer splits). Every call on one GPU shares that GPU's array: calls that overlap on one GPU
- * (concurrent streams or threads) race and must be serialised by the caller. */
+/* Allocation-free variant of cf_kv_paged_attention_batched_async: the partials go to a library-owned device array of
+ * CF_KV_BATCHED_NOALLOC_SCRATCH_BYTES per GPU instead of desc->workspace (ignored). No counterpart in the reference; it
+ * is for callers that cannot allocate device memory (code under HIP graph capture, tight serving loops, harnesses that
+ * forbid hipMalloc). It calls no allocator. The launches, and so every bit of the results, are those of the workspace
+ * entry point, except where that one runs spans (splits = 0) and this one runs splits: where the split launch needs no
+ * partials (one split; such calls may overlap here), or the span states exceed the array. The results of the two then
+ * differ in fp32 rounding. A descriptor whose split partials exceed the array returns CF_ERR_UNSUPPORTED (use the
+ * workspace entry point, or fewer splits). Every call on one GPU shares that GPU's array: calls that overlap on one GPU
+ * (concurrent streams or threads) and use it race and must be serialised by the caller. */
 #define CF_KV_BATCHED_NOALLOC_SCRATCH_BYTES (8u << 20)
 cf_status cf_kv_paged_attention_batched_noalloc_async(const cf_kv_batched_desc *desc, void *stream);
 

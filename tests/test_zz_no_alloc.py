@@ -104,3 +104,33 @@ def test_noalloc_refuses_partials_beyond_the_array(dev):
     assert L.cf_kv_batched_workspace_bytes(C.byref(huge)) > 8 << 20
     L.cf_kv_paged_attention_batched_noalloc_async.restype = C.c_int32
     assert L.cf_kv_paged_attention_batched_noalloc_async(C.byref(huge), None) == A.CF_ERR_UNSUPPORTED
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_noalloc_spans(dev, D):
+    """Batches that the workspace entry point runs as spans: the same launch here where the split launch would use the
+    array as well, the split launch where that needs no partials."""
+    import torch
+    heads = 8
+    state = 4 * (D + 2) * 4
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    span_bytes = lambda S: (4 * (S + 1) + 255) // 256 * 256 + heads * (cus // heads * 12 + S) * state  # noqa: E731
+    lens = [8200, 300, 64, 1, 700, 129, 2000, 90, 500, 65, 17, 256]
+    print(f"case E: 12 ragged sequences, 2 splits otherwise, hd {D}", flush=True)
+    kvb, q, qp = _case(dev, lens, heads, D, seed=310)
+    ref, got, need = _both(kvb, q, qp, 0)
+    assert need == span_bytes(len(lens)) <= 8 << 20
+    assert torch.isfinite(ref).all() and torch.equal(ref, got)
+    lens = [3100, 40, 900, 64] * 8
+    print(f"case F: 32 ragged sequences, one split otherwise, hd {D}", flush=True)
+    kvb, q, qp = _case(dev, lens, heads, D, seed=311, codec=1)
+    ref, got, need = _both(kvb, q, qp, 0)
+    assert need == span_bytes(len(lens))
+    split = torch.full_like(q, float("nan"))
+    d = kvb.desc(q, split, qp, 1.0 / np.sqrt(D))
+    d.workspace, d.workspace_bytes = None, 0
+    kvb.attention(q, split, qp, 1.0 / np.sqrt(D), desc=d)
+    torch.cuda.synchronize()
+    assert torch.isfinite(got).all() and torch.equal(got, split)
+    # the same sums grouped otherwise (see the spans' own test)
+    assert float(((ref - got).norm(dim=-1) / got.norm(dim=-1)).max()) <= 1e-5
