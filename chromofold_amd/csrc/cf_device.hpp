@@ -24,6 +24,21 @@ inline unsigned grid_for(size_t work, unsigned per_block) {
   return static_cast<unsigned>((work + per_block - 1) / per_block);
 }
 
+// Compute units of the current device, read once per host thread and device (256 where there is none).
+inline uint32_t cu_count() {
+  static thread_local int cached_dev = -1;
+  static thread_local uint32_t cached = 0;
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return 256;
+  if (dev != cached_dev) {
+    int cus = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
+    cached = static_cast<uint32_t>(cus);
+    cached_dev = dev;
+  }
+  return cached;
+}
+
 // ------------------------------------------------------------------------------------------------ RRR constants
 // T = 15-bit blocks, S = 64 blocks per rank superblock, K = 32 superblocks per int32 anchor. These are baked into
 // the .cfrw/.cffm formats (reference include/chromofold/detail/rrr_wavelet_device.cuh:16-18).

@@ -2017,21 +2017,6 @@ __global__ CF_KV_OCC __launch_bounds__(64 * kWavesNarrow) void seam_group_kernel
   }
 }
 
-// CUs of the current device (cached per thread and device).
-uint32_t cu_count() {
-  static thread_local int cached_dev = -1;
-  static thread_local uint32_t cached = 0;
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return 256;
-  if (dev != cached_dev) {
-    int cus = 0;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
-    cached = static_cast<uint32_t>(cus);
-    cached_dev = dev;
-  }
-  return cached;
-}
-
 // Launch shape of kv_batched_kernel: context splits per (sequence, KV head) and wavefronts per workgroup.
 // Narrow (4 wavefronts, three workgroups per CU) is the base shape. Issue arbitration favours the oldest wavefronts,
 // so the three workgroups of a CU finish far apart; when the grid is one round of workgroups (fewer units than three
@@ -2074,7 +2059,7 @@ constexpr uint32_t kWidePairsPerWave = 2;
 BatchedPlan split_plan(const cf_kv_batched_desc *d) {
   const uint32_t units = d->seq_count * d->kv_head_count;
   const uint32_t pairs = (d->max_groups + 1) / 2;
-  const uint32_t cus = cu_count();
+  const uint32_t cus = cfd::cu_count();
   auto wide_ok = [&](uint32_t s) { return pairs / s >= kWidePairsPerWave * kWavesWide; };
   const uint32_t resident = 3 * cus;
   if (d->splits) return {d->splits, units * d->splits <= cus && wide_ok(d->splits) ? 12u : 4u, 0u};
@@ -2088,13 +2073,13 @@ BatchedPlan split_plan(const cf_kv_batched_desc *d) {
 }
 
 uint32_t span_workgroups(uint32_t heads) {
-  return std::min<uint32_t>(std::max<uint32_t>(1, cu_count() / heads), kSpanMaxWg);
+  return std::min<uint32_t>(std::max<uint32_t>(1, cfd::cu_count() / heads), kSpanMaxWg);
 }
 
 BatchedPlan batched_plan(const cf_kv_batched_desc *d) {
   const BatchedPlan p = split_plan(d);
   if (d->splits != 0 || d->seq_count < 2 || d->seq_count > kSpanMaxSeqs ||
-      static_cast<uint64_t>(d->seq_count) * d->kv_head_count >= 3u * cu_count())
+      static_cast<uint64_t>(d->seq_count) * d->kv_head_count >= 3u * cfd::cu_count())
     return p;
   const uint32_t pairs = (d->max_groups + 1) / 2, lanes = p.splits * p.waves;  // wavefronts of the longest context
   if (pairs < 2 * lanes) return p;
@@ -2124,7 +2109,7 @@ struct CascadePlan {
 CascadePlan cascade_plan(const cf_kv_batched_desc *d, uint32_t shared) {
   CascadePlan p{};
   const uint32_t tiles = ((d->seq_count + 15) / 16) * d->kv_head_count;
-  const uint32_t want = std::max<uint32_t>(1, (2 * cu_count() + tiles - 1) / tiles);
+  const uint32_t want = std::max<uint32_t>(1, (2 * cfd::cu_count() + tiles - 1) / tiles);
   p.psplits = std::min<uint32_t>(want, shared);
   cf_kv_batched_desc rest = *d;
   rest.max_groups = std::max<uint32_t>(1, d->max_groups - shared);
@@ -2320,7 +2305,7 @@ uint32_t seam_route_splits(const cf_kv_paged_attention_desc &d) {
   // about two pages per wavefront, within one round of workgroups (three per CU)
   const uint32_t per_head = (d.page_count + d.kv_head_count - 1) / d.kv_head_count;
   uint32_t s = std::max<uint32_t>(1, per_head / (2 * kWavesNarrow));
-  s = std::min<uint32_t>(s, std::max<uint32_t>(1, 3 * cu_count() / d.kv_head_count));
+  s = std::min<uint32_t>(s, std::max<uint32_t>(1, 3 * cfd::cu_count() / d.kv_head_count));
   return std::min<uint32_t>(s, 64);
 }
 

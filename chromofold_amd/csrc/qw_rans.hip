@@ -3,20 +3,20 @@
 // coded form.
 //
 // One 1024-thread workgroup (16 waves) owns one band of 16 rows and walks K in chunks of 16 stripes (4096 columns);
-// wave w decodes stripe w of the chunk, its 64 lanes being the stripe's 64 interleaved rANS states (the code also
-// runs 8 waves of two stripes each, decoded together as two chains per lane: measured slower, 9.9 against 9.1 us at
-// B = 1):
+// wave w decodes stripe w of the chunk, its 64 lanes being the stripe's 64 interleaved rANS states (8 waves of two
+// stripes each, decoded together as two chains per lane, were slower: 9.9 against 9.1 us at B = 1):
 //   stage    the chunk's slot (fixed size, so its address needs no offset read) is loaded with straight-line 16-byte
-//            loads together with the lane states, the stripe offsets, the scales and the first x fragments;
+//            loads together with the lane states, the stripe offsets, the scales and (whole stripes) the first x
+//            fragments; with several chunks, the next one's while the one before it is decoded;
 //   table    while those loads are in flight the band's 256 cumulative starts become a 4096-entry LDS table:
 //            slot -> {f | (slot - cum) << 16, the pair's two weights as bf16 (sym - zero, exact)};
 //   decode   32 steps per lane: table lookup, x = f * (x >> 12) + slot - cum, and a 16-bit renormalisation word
 //            for the lanes whose state fell below 2^16, taken from the staged stream at a wave-uniform cursor plus
 //            the lane's rank among the lanes that need one (ballot / mbcnt);
-//   MFMA     every two steps give a lane 4 consecutive weights of its row: the B operand of one
-//            v_mfma_f32_16x16x16_bf16 (lane 16 g + r: row r, k = 4 g..4 g + 3). The stripe's column order puts the
+//   MFMA     every four steps give a lane 8 consecutive weights of its row: the B operand of one
+//            v_mfma_f32_16x16x32_bf16 (lane 16 g + r: row r, k = 8 g..8 g + 7). The stripe's column order puts the
 //            same lane's x values in the A operand, so decoded weights never leave the registers; each 64-column
-//            segment's 4 MFMAs accumulate apart and the segment's scale multiplies them once;
+//            segment's 2 MFMAs accumulate apart and the segment's scale multiplies them once;
 //   reduce   the waves' partial tiles are summed through LDS in a fixed order and y is written once.
 // Batches above 64 rows run as several launches of up to 4 tiles each.
 #include <hip/hip_runtime.h>
@@ -105,8 +105,9 @@ __device__ void build_table(uint2 cw, int zero, uint2 *__restrict__ tab, uint32_
   }
 }
 
-// 8 bf16 of x row b from column c (one 16-byte unit), zero for a row past the batch or a column past K: the A
-// operands of two MFMAs of lane group g (the general path; FAST loads 16 bytes straight from x).
+// 8 bf16 of x row b from column c (one 16-byte unit), zero for a row past the batch or a column past K: the A operand
+// of one MFMA for the lane's group (the general path; FAST loads 16 bytes straight from x). Loaded where it is used:
+// 4000 x 4500 columns took 20.9 / 43.8 / 107.7 us at 1 / 16 / 48 rows, 22.9 / 47.7 / 108.0 with loads further ahead.
 __device__ __forceinline__ uint4 x_frag8(const uint16_t *__restrict__ x, int b, int B, int c, int K) {
   uint32_t v[8];
 #pragma unroll
@@ -364,25 +365,11 @@ qw_rans_kernel(RansArgs a) {
   }
 }
 
-uint32_t cu_count() {  // multiprocessors of the current device, per host thread
-  static thread_local int cached_dev = -1;
-  static thread_local uint32_t cached = 0;
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return 256;
-  if (dev != cached_dev) {
-    int cus = 0;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
-    cached = static_cast<uint32_t>(cus);
-    cached_dev = dev;
-  }
-  return cached;
-}
-
 template <int NT, bool FAST, int XR, bool PIPE>
 void launch_rans_sl(const RansArgs &a, unsigned grid, hipStream_t s) {
   // Two workgroups fit a CU in some variants. A grid of at most one per CU gets LDS that keeps them apart: the
   // dispatcher otherwise puts pairs of them on one CU while others idle (4096 x 4096, one row: 9.6 against 8.2 us).
-  const unsigned apart = grid <= cu_count() ? 20480u : 0u;
+  const unsigned apart = grid <= cfd::cu_count() ? 20480u : 0u;
   if (max(a.chunk_words, a.last_words) <= 2 * kThreads * 8)
     qw_rans_kernel<NT, FAST, 2, XR, PIPE><<<grid, kThreads, apart, s>>>(a);
   else
