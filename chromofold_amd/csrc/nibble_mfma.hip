@@ -501,12 +501,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
       mx[j] = sc[j];
     }
     row_max4(mx);
-    // V scales in the accumulators' unit: a weight p * v_scale * 2^vunit stays below 2^15
+    // V scales in the accumulators' unit: a weight p * v_scale * 2^vunit stays below 2^15 (by magnitude: the scales of
+    // pages that a caller publishes may be negative)
     float vs[NB], vmax = 0.0f;
 #pragma unroll
     for (int s = 0; s < NB; ++s) {
       vs[s] = n_vs[s] * vfac;
-      vmax = fmaxf(vmax, vs[s]);
+      vmax = fmaxf(vmax, __builtin_fabsf(vs[s]));
     }
     // raise the running maxima and the unit (and rescale the accumulators) only when some lane's grew
     bool grow = vmax >= kWeightTop;
@@ -515,7 +516,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     if (__ballot(grow) != 0) {
       float top = 0.0f;
 #pragma unroll
-      for (int s = 0; s < NB; ++s) top = fmaxf(top, n_vs[s]);
+      for (int s = 0; s < NB; ++s) top = fmaxf(top, __builtin_fabsf(n_vs[s]));
       const int un = min(vunit, max(15 - __builtin_amdgcn_frexp_expf(cfd::row16_max(top)), -kUnitMax)), du = un - vunit;
       vunit = un;
       vfac = ldexpf(1.0f, un);

@@ -58,3 +58,73 @@ def test_v_magnitudes(bs):
     res.reclaim()
     res.close()
     eng.close()
+
+
+@pytest.mark.parametrize("mode", ["resolver32", "resolver64", "resolver128", "runtime"])
+def test_negative_v_scales(mode):
+    """Pages a caller publishes with scales of its own: V scales of either sign and of several magnitudes, all of them
+    negative among others."""
+    import torch
+    from chromofold_amd import sealkv as S
+    dev, kvh, gqa, page, D = torch.device("cuda:0"), 2, 4, 32, 128
+    print(f"case {mode}", flush=True)
+    rng = np.random.default_rng(11)
+    keep = []
+
+    def up(a):
+        keep.append(torch.from_numpy(np.ascontiguousarray(a)).to(dev))
+        return keep[-1]
+
+    flips = [lambda v: -np.abs(v), lambda v: np.where(rng.random(v.shape) < 0.5, -v, v).astype(np.float32)]
+    mags = [[1.0] * 5, [1e-3] * 33, [1e3] * 5, [1e4, 1e-4] * 4]
+    q = rng.standard_normal((1, kvh * gqa, D)).astype(np.float32)
+    outs, refs = [], []
+    if mode == "runtime":
+        bs = 32
+        rt = S.AttentionRuntime(1, kvh, kvh * gqa, D, gqa=gqa, page_size=page, block_size=bs)
+        items = (S.cf_attention_batch_item * (len(flips) * len(mags)))()
+    else:
+        bs = int(mode[8:])
+        res, batch = S.MsResolver(1, kvh, kvh * gqa, D, page), []
+    for i, (flip, mag) in enumerate((f, m) for f in flips for m in mags):
+        descs, host = (S.cf_device_page_descriptor * len(mag))(), []
+        for p, amp in enumerate(mag):
+            k, v = (rng.standard_normal((page, kvh, D)).astype(np.float32) for _ in range(2))
+            v *= np.float32(amp)
+            if mode == "runtime":
+                (kp, ks), (vp, vs) = O.rt_quantize(k, bs), O.rt_quantize(v, bs)
+                vs = flip(vs)
+                host.append(O.RtPage(kp, vp, ks, vs, p * page, page, D, bs))
+            else:
+                s = O.nib_seal_page(k, v, p * page, bs)
+                kp, ks, vp, vs = s.k_payload, s.k_scales, s.v_payload, flip(s.v_scales)
+                host.append(O.NibPage(kp, vp, ks, vs, p * page, page))
+            d = descs[p]
+            d.key_payload, d.value_payload, d.key_scales, d.value_scales = (up(a).data_ptr() for a in (kp, vp, ks, vs))
+            d.token_begin, d.token_count, d.kv_head_count, d.head_dim, d.block_size = p * page, page, kvh, D, bs
+        qpos, out = len(mag) * page - 1, torch.full((1, kvh * gqa, D), float("nan"), device=dev)
+        outs.append(out)
+        if mode == "runtime":
+            it, qd = items[i], up(q)
+            it.sequence_id, it.layer = 100 + i, 0
+            it.query = S.cf_device_tensor_view(qd.data_ptr(), S._TYPE[qd.dtype], 1, kvh * gqa, D, 0, 4 * D, 4, 0)
+            it.output, it.output_type = out.data_ptr(), S._TYPE[out.dtype]
+            it.output_token_stride_bytes, it.output_head_stride_bytes, it.output_element_stride_bytes = 0, 4 * D, 4
+            it.query_token_begin, it.softmax_scale, it.causal_window = qpos, 0.09, 0
+            it.sealed_pages = up(np.frombuffer(bytearray(descs), np.uint8)).data_ptr()
+            it.sealed_page_count = len(mag)
+            refs.append(O.rt_attention_f64(q[0], kvh, gqa, qpos, 0, it.softmax_scale, host, None, None, 0))
+        else:
+            res.create(i)
+            for d in descs:
+                res.publish(i, 0, d)
+            batch.append((i, 0, up(q), out, qpos, 0.09, 0))
+            refs.append(O.nib_attention(host, bs, q, qpos, kvh, gqa, 0.09, 0))
+    rt.execute(items) if mode == "runtime" else res.execute(batch)
+    torch.cuda.synchronize()
+    for i, (out, ref) in enumerate(zip(outs, refs)):
+        got, ref = out.cpu().numpy().astype(np.float64).reshape(-1, D), ref.astype(np.float64).reshape(-1, D)
+        assert np.isfinite(got).all(), i
+        err = np.linalg.norm(got - ref, axis=-1) / np.linalg.norm(ref, axis=-1)
+        assert err.max() <= 2.0 ** -19, (i, float(err.max()))
+    rt.close() if mode == "runtime" else (res.reclaim(), res.close())
