@@ -465,7 +465,9 @@ __device__ __forceinline__ uint32_t span_owner(uint32_t x, uint32_t pairs, uint3
 }
 
 // AFTER: the workgroup is the only one of a cascade row and finishes it with the prefix states of slots 0 .. slot0 - 1
-// (a kernel of its own: in the ordinary one that code costs a single sequence's decode 0.3 of 17.2 us).
+// (a kernel of its own: in the ordinary one that code costs a single sequence's decode 0.3 of 17.2 us). At most
+// kAfterStates of them, each thread's values in one memory latency; see cascade_after.
+constexpr uint32_t kAfterStates = 8;
 template <int D, int CODEC, int W, bool AFTER = false>
 __global__ CF_KV_OCC __launch_bounds__(64 * W) void kv_batched_kernel(cf_kv_batched_desc d, uint32_t splits,
                                                                        float *__restrict__ partial, SplitSlots ss) {
@@ -694,6 +696,24 @@ __global__ CF_KV_OCC __launch_bounds__(64 * W) void kv_batched_kernel(cf_kv_batc
     gi = gn;
   }
 
+  // AFTER: the prefix states, all in flight during the reduction of the own groups
+  constexpr int kIt = AFTER ? (kGqa * D + kThreads - 1) / kThreads : 1;
+  float pm[kIt][kAfterStates], pl[kIt][kAfterStates], po[kIt][kAfterStates];
+  if constexpr (AFTER) {
+    const float *pp = partial + (static_cast<size_t>(seq) * d.kv_head_count + head) * ss.slots * (kGqa * (D + 2));
+#pragma unroll
+    for (int it = 0; it < kIt; ++it) {
+      const int i = min(static_cast<int>(threadIdx.x) + it * kThreads, kGqa * D - 1);
+#pragma unroll
+      for (uint32_t u = 0; u < kAfterStates; ++u) {
+        const float *q = pp + min(u, ss.slot0 - 1) * (kGqa * (D + 2)) + (i / D) * (D + 2);
+        pm[it][u] = q[D];
+        pl[it][u] = q[D + 1];
+        po[it][u] = q[i % D];
+      }
+    }
+  }
+
   // ---- reduce the wavefront: sum the hi and lo parts (lanes t and t + 16; lanes 32-63 hold the repeated rows
   // 8-15) in absolute units, l over all lanes
 #pragma unroll
@@ -724,16 +744,15 @@ __global__ CF_KV_OCC __launch_bounds__(64 * W) void kv_batched_kernel(cf_kv_batc
   __syncthreads();
 
   // ---- merge the wavefronts; write the split partial (or the final output when splits == 1)
-  for (int i = threadIdx.x; i < kGqa * D; i += kThreads) {
-    const int h = i / D, dd = i % D;
-    float m = -INFINITY;
-    bool nan = false;
+  auto merge_waves = [&](int h, int dd, float &m, float &l, float &o, bool &nan) {
+    m = -INFINITY;
+    nan = false;
     for (int w = 0; w < W; ++w) {
       const float mw = reinterpret_cast<const float *>(s_buf[w])[h * (D + 2) + D];
       nan |= mw != mw;
       m = fmaxf(m, mw);
     }
-    float l = 0.0f, o = 0.0f;
+    l = o = 0.0f;
     if (m != -INFINITY)
       for (int w = 0; w < W; ++w) {
         const float *rw = reinterpret_cast<const float *>(s_buf[w]);
@@ -743,44 +762,29 @@ __global__ CF_KV_OCC __launch_bounds__(64 * W) void kv_batched_kernel(cf_kv_batc
         l += rw[h * (D + 2) + D + 1] * sc;
         o += rw[h * (D + 2) + dd] * sc;
       }
-    if (nan) m = __builtin_nanf("");
-    if (!AFTER && ss.slots == 1) {
-      if (static_cast<uint32_t>(h) < gqa)
-        d.output[(static_cast<size_t>(seq) * d.query_head_count + head * gqa + h) * D + dd] =
-            nan ? m : l > 0.0f ? o / l : 0.0f;
-    } else if (AFTER) {
-      // the merge kernel's order and rules, beside the other workgroups' decode
-      const float *pp = partial + (static_cast<size_t>(seq) * d.kv_head_count + head) * ss.slots * (kGqa * (D + 2)) + h * (D + 2);
-      constexpr uint32_t kB = 4;
+  };
+  if constexpr (AFTER) {  // the merge kernel's order and rules
+#pragma unroll
+    for (int it = 0; it < kIt; ++it) {
+      const int i = threadIdx.x + it * kThreads, h = i / D, dd = i % D;
+      if (i >= kGqa * D) break;
+      float m, l, o;
+      bool nan;
+      merge_waves(h, dd, m, l, o, nan);
       float mm = m;
-      for (uint32_t s0 = 0; s0 < ss.slot0; s0 += kB) {
-        float ms[kB];
 #pragma unroll
-        for (uint32_t u = 0; u < kB; ++u) ms[u] = pp[min(s0 + u, ss.slot0 - 1) * (kGqa * (D + 2)) + D];
-#pragma unroll
-        for (uint32_t u = 0; u < kB; ++u) {
-          nan |= ms[u] != ms[u];
-          mm = fmaxf(mm, ms[u]);
-        }
+      for (uint32_t u = 0; u < kAfterStates; ++u) {  // (past the last state: the last one again)
+        nan |= pm[it][u] != pm[it][u];
+        mm = fmaxf(mm, pm[it][u]);
       }
       float lt = 0.0f, ot = 0.0f;
       if (mm != -INFINITY) {
-        for (uint32_t s0 = 0; s0 < ss.slot0; s0 += kB) {
-          float mq[kB], lq[kB], oq[kB];
 #pragma unroll
-          for (uint32_t u = 0; u < kB; ++u) {
-            const float *q = pp + min(s0 + u, ss.slot0 - 1) * (kGqa * (D + 2));
-            mq[u] = q[D];
-            lq[u] = q[D + 1];
-            oq[u] = q[dd];
-          }
-#pragma unroll
-          for (uint32_t u = 0; u < kB; ++u) {
-            if (s0 + u >= ss.slot0 || mq[u] == -INFINITY) continue;
-            const float sc = __expf(mq[u] - mm);
-            lt += lq[u] * sc;
-            ot += oq[u] * sc;
-          }
+        for (uint32_t u = 0; u < kAfterStates; ++u) {
+          if (u >= ss.slot0 || pm[it][u] == -INFINITY) continue;
+          const float sc = __expf(pm[it][u] - mm);
+          lt += pl[it][u] * sc;
+          ot += po[it][u] * sc;
         }
         if (m != -INFINITY) {
           const float sc = __expf(m - mm);
@@ -791,6 +795,19 @@ __global__ CF_KV_OCC __launch_bounds__(64 * W) void kv_batched_kernel(cf_kv_batc
       if (static_cast<uint32_t>(h) < gqa)
         d.output[(static_cast<size_t>(seq) * d.query_head_count + head * gqa + h) * D + dd] =
             nan ? __builtin_nanf("") : lt == 0.0f ? 0.0f : ot / lt;
+    }
+    return;
+  }
+  for (int i = threadIdx.x; i < kGqa * D; i += kThreads) {
+    const int h = i / D, dd = i % D;
+    float m, l, o;
+    bool nan;
+    merge_waves(h, dd, m, l, o, nan);
+    if (nan) m = __builtin_nanf("");
+    if (ss.slots == 1) {
+      if (static_cast<uint32_t>(h) < gqa)
+        d.output[(static_cast<size_t>(seq) * d.query_head_count + head * gqa + h) * D + dd] =
+            nan ? m : l > 0.0f ? o / l : 0.0f;
     } else {
       float *pp = partial + ((static_cast<size_t>(seq) * d.kv_head_count + head) * ss.slots + ss.slot0 + split) *
                                 (kGqa * (D + 2));
@@ -2118,6 +2135,16 @@ CascadePlan cascade_plan(const cf_kv_batched_desc *d, uint32_t shared) {
   return p;
 }
 
+// Whether the workgroups of the own groups finish their rows (kv_batched_kernel's AFTER) or the merge launch does: few
+// prefix states fit a thread's registers and arrive in one latency, beside the own groups' reduction. us with the row's own
+// workgroup / with the merge launch, 8 KV / 32 query heads, own tokens at most `own`:
+//   40 sequences, 8 states, own 128     24.1 / 28.7      128, 8 states, own 200     60.0 / 66.3
+//   100, 2 states, own 128              33.7 / 36.4      200, 5 states, own 200    104.6 / 108.1
+//   100, 8 states, own 200              41.5 / 47.4      256, 4 states, own 512    150.7 / 154.7
+// More states in batches of four, two latencies a batch and element: 10 states 73.6 / 69.6 (100 sequences), 16 29.3 / 28.0,
+// 32 34.9 / 27.9, 48 48.4 / 36.6 (16 sequences).
+bool cascade_after(const CascadePlan &p) { return p.suffix.splits == 1 && p.psplits <= kAfterStates; }
+
 template <int D>
 void launch_span(const cf_kv_batched_desc &d, uint32_t nwg, void *ws, hipStream_t s) {
   const SpanArgs sp{nwg, static_cast<uint32_t *>(ws)};
@@ -2232,7 +2259,7 @@ extern "C" cf_status cf_kv_paged_attention_cascade_async(const cf_kv_batched_des
   const SplitSlots rest{shared_groups, p.psplits, p.slots};
   const dim3 grid(p.suffix.splits, d->kv_head_count, d->seq_count);
   const bool rans = d->codec == CF_KV_CODEC_RANS_HYBRID;
-  if (p.suffix.splits == 1) {
+  if (cascade_after(p)) {
     if (rans) launch_batched<128, CF_KV_CODEC_RANS_HYBRID, true>(*d, p.suffix, grid, ws, rest, s);
     else launch_batched<128, CF_KV_CODEC_INT8, true>(*d, p.suffix, grid, ws, rest, s);
     return cfd::launch_status();

@@ -22,6 +22,18 @@ def _dequant(x):
 @pytest.mark.parametrize("splits", [1, 3])
 @pytest.mark.parametrize("H,gqa,shared,S", [(8, 4, 8, 5), (3, 2, 13, 17), (1, 3, 40, 33), (5, 1, 5, 16), (2, 4, 70, 1)])
 def test_prefix_pass_against_float64(H, gqa, shared, S, splits):
+    _check(H, gqa, shared, S, splits, [1, 17, 64, 200])
+
+
+@pytest.mark.parametrize("shared", [1, 7, 8, 9])
+@pytest.mark.parametrize("own", [[1, 200], [3100, 3300]])
+def test_prefix_states_of_one_workgroup(shared, own):
+    """Rows of one workgroup with as many prefix states as it adds itself (1 to 8, one per group here) and one more, which
+    takes the merge launch; 4 wavefronts per workgroup, and 12."""
+    _check(2, 3, shared, 5, 1, own)
+
+
+def _check(H, gqa, shared, S, splits, own_lens):
     import torch
     from chromofold_amd import kv
     print(f"case H={H} gqa={gqa} shared={shared} S={S} splits={splits}", flush=True)
@@ -30,7 +42,7 @@ def test_prefix_pass_against_float64(H, gqa, shared, S, splits):
     q = rng.standard_normal((S, H * gqa, D)).astype(np.float32)
     common = rng.standard_normal((H, D)).astype(np.float32)
     q += 0.3 * np.repeat(common, gqa, 0)  # the ramp of the keys along `common` raises every row's scores
-    lens = [n + int(rng.choice([1, 17, 64, 200])) for _ in range(S)]
+    lens = [n + int(rng.choice(own_lens)) for _ in range(S)]
     pos = [t - 1 for t in lens]
     pos[S // 2] = n // 2 + 5  # inside the prefix
     pos[-1] = lens[-1] - 1 if S > 1 else n - 64
@@ -38,7 +50,7 @@ def test_prefix_pass_against_float64(H, gqa, shared, S, splits):
     vexp = np.repeat(rng.choice([-9, -1, 0, 1, 2, 3, 8], shared), 64).astype(np.float32)
     k0 = rng.standard_normal((H, n, D)).astype(np.float32) + (ramp[:, None] * common[:, None, :]).astype(np.float32)
     v0 = rng.standard_normal((H, n, D)).astype(np.float32) * np.exp2(vexp)[:, None]
-    v0[:, 64:128] = 0.0
+    v0[:, 64:128] = 0.0  # (nothing where the prefix is one group)
     data = []
     for T in lens:
         own = [rng.standard_normal((H, T - n, D)).astype(np.float32) for _ in range(2)]
