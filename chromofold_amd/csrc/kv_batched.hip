@@ -2064,6 +2064,15 @@ __global__ CF_KV_OCC __launch_bounds__(64 * kWavesNarrow) void seam_group_kernel
 //     tokens);
 //   * tables with room for so few groups that the splits leave less than two chain pairs per wavefront: there is little
 //     to balance, and prologue and merge cost 3 us (20 x 2000 tokens: 26.9 against 29.6 us, 32 x 300: 15.0 against 18.4);
+//   * one split of 4 wavefronts (more than 1.5 units per CU) with less than six chain pairs per wavefront of INT8 groups, from
+//     two units per CU also with less than four of rANS groups: the units fill the CUs evenly by themselves and need no
+//     merge, where a span's 12 wavefronts round their pairs up. 8 KV heads, spans against splits, us, for equal lengths,
+//     lengths from half the longest and lengths from 1/40 of it:
+//       rANS hd 128  80 x 900    41.7, 37.7                                80 x 2048  77.3, 73.8   55.5, 66.1   40.3, 59.2
+//                    95 x 1500   66.5, 57.3   53.7, 52.2   37.2, 46.1      64 x 4096 120.7, 117.9  94.9, 111.0  45.7, 80.7
+//       INT8 hd 64   64 x 1500   25.0, 18.3   22.1, 16.0   16.3, 13.8      64 x 4096  56.1, 59.2   40.3, 38.0   23.7, 28.5
+//            hd 128  95 x 2048   79.6, 67.0   63.1, 57.5   34.7, 39.1      95 x 4096 138.8, 125.1 103.7, 107.5  55.1, 71.1
+//     (below the lines batches of like lengths lose more than ragged ones gain);
 //   * larger grids: one workgroup per unit, which the dispatcher balances and whose neighbours share a common prefix in
 //     L1;
 //   * callers who fix the splits, or whose workspace is too small for the span states.
@@ -2099,7 +2108,12 @@ BatchedPlan batched_plan(const cf_kv_batched_desc *d) {
       static_cast<uint64_t>(d->seq_count) * d->kv_head_count >= 3u * cfd::cu_count())
     return p;
   const uint32_t pairs = (d->max_groups + 1) / 2, lanes = p.splits * p.waves;  // wavefronts of the longest context
-  if (pairs < 2 * lanes) return p;
+  uint32_t least = 2;
+  if (p.splits == 1 && p.waves == kWavesNarrow) {  // more than 1.5 whole units per CU
+    if (d->codec == CF_KV_CODEC_INT8) least = 6;
+    else if (d->seq_count * d->kv_head_count >= 2 * cfd::cu_count()) least = 4;
+  }
+  if (pairs < least * lanes) return p;
   return {1u, 12u, span_workgroups(d->kv_head_count)};
 }
 

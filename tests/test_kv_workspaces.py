@@ -101,3 +101,18 @@ def test_prepared_descriptors_on_the_gpu():
     torch.cuda.synchronize()
     for o, w in zip(got, want):
         assert torch.equal(o, w)
+
+
+@pytest.mark.parametrize("codec,S,groups,spans", [
+    ("int8", 95, 46, False), ("int8", 95, 47, True), ("int8", 49, 46, False), ("int8", 49, 47, True),
+    ("rans", 64, 30, False), ("rans", 64, 31, True), ("rans", 63, 14, False), ("rans", 63, 15, True)])
+def test_which_full_grids_run_as_spans(codec, S, groups, spans):
+    """Batches of 8 heads with more than 1.5 units per CU (256 CUs where no GPU says otherwise), which hold no workspace as
+    one split: spans from six chain pairs per wavefront of INT8 groups; of rANS groups from two, from 64 sequences (two units
+    per CU) on from four."""
+    kv, b, q, o, pos = _host_batch(S=S, groups=groups)
+    if codec == "rans":
+        import torch
+        b.codec, b.tables = kv.CODEC_RANS_HYBRID, torch.zeros(16 * kv.TABLE_BYTES, dtype=torch.uint8)
+    d = b.desc(q, o, pos, 0.1, stream=_Stream(1))
+    assert (d.workspace_bytes > 0) == spans
